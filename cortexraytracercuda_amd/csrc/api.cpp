@@ -176,6 +176,7 @@ int Context::init(const crt_config* cfg) {
     stack_lds = config.stack_lds ? config.stack_lds : 16u;
     if (config.ray_sort > 2) return set_error(CRT_ERR_INVALID_ARGUMENT, "unknown ray_sort");
     ray_sort = config.ray_sort == 1u ? 1u : 0u;
+    staged = config.extend_kernel != 0 || ray_sort != 0 || config.count_work != 0;
     if (config.bvh_builder > CRT_BVH_DEVICE) return set_error(CRT_ERR_INVALID_ARGUMENT, "unknown bvh_builder");
     bvh_builder = config.bvh_builder ? config.bvh_builder : (uint32_t)CRT_BVH_HOST;
     if (config.serve_order > CRT_SERVE_ROUND_ROBIN) return set_error(CRT_ERR_INVALID_ARGUMENT, "unknown serve_order");
@@ -193,6 +194,7 @@ int Context::init(const crt_config* cfg) {
     if ((rc = scene_table.alloc(sizeof(crt_dev_scene) * kMaxScenes, this))) return rc;
     if ((rc = counters.alloc(sizeof(crt_dev_counters), this))) return rc;
     if ((rc = ctl.alloc(sizeof(uint32_t) * 2 * CRT_CTL_WORDS * kMaxSubPasses, this))) return rc;
+    if ((rc = path_next.alloc(sizeof(uint32_t) * kMaxPassRequests, this))) return rc;
     HIP_TRY(hipHostMalloc((void**)&ctl_host, sizeof(uint32_t) * CRT_CTL_WORDS * kCtlRing * kMaxSubPasses,
                           hipHostMallocDefault));
     for (int k = 0; k < kCtlRing * kMaxSubPasses; ++k) HIP_TRY(hipEventCreateWithFlags(&ctl_ev[k], hipEventDisableTiming));
@@ -248,6 +250,7 @@ int Context::scratch_bufs(PassBufs& B) {
     B.out_rad = (float4*)take(P * 16);
     B.ctl = (uint32_t*)take(2 * CRT_CTL_WORDS * sizeof(uint32_t));
     B.counters = (crt_dev_counters*)take(sizeof(crt_dev_counters));
+    B.next = (uint32_t*)take(sizeof(uint32_t));
     B.req[0] = (crt_dev_request*)take(sizeof(crt_dev_request));
     B.req[1] = (crt_dev_request*)take(sizeof(crt_dev_request));
     if (off >= scratch_bytes) return set_error(CRT_ERR_INTERNAL, "scratch array too small for the pass state");
@@ -259,7 +262,9 @@ int Context::scratch_bufs(PassBufs& B) {
     B.slots = (uint32_t)S;
     B.pass_ids = (uint32_t)P;
     B.extend_grid = (uint32_t)grid;
+    B.gstack_words = grid * per_block_stack / sizeof(uint32_t);
     B.max_sub = 1;
+    B.max_requests = 1;
     return CRT_OK;
 }
 
@@ -312,6 +317,9 @@ PassBufs Context::pool_bufs() {
     }
     B.hit = (float4*)hit.p; B.hit_inst = (uint32_t*)hit_inst.p; B.out_rad = (float4*)out_rad.p;
     B.gstack = (uint32_t*)gstack.p; B.ctl = (uint32_t*)ctl.p; B.counters = (crt_dev_counters*)counters.p;
+    B.next = (uint32_t*)path_next.p;
+    B.gstack_words = gstack.bytes / sizeof(uint32_t);
+    B.max_requests = kMaxPassRequests;
     B.slots = std::min(max_paths, path_capacity);
     B.pass_ids = pass_capacity;
     B.extend_grid = extend_grid;
@@ -625,6 +633,21 @@ bool Job::take(uint32_t cap, WorkItem& w) {
     return true;
 }
 
+bool Job::take_whole(uint32_t cap, WorkItem& w) {
+    if (rd.rng_mode != CRT_RNG_MINSTD) return take(cap, w);
+    if (s_next >= s_end || cap == 0) return false;
+    w.job = this;
+    w.pix_begin = p_next; w.pix_count = std::min(cap, npix - p_next);
+    w.sample_begin = s_next; w.sample_count = s_end - s_next;
+    p_next += w.pix_count;
+    if (p_next == npix) { p_next = 0; s_next = s_end; }
+    return true;
+}
+
+uint32_t WorkItem::whole_ids() const {
+    return job->rd.rng_mode == CRT_RNG_MINSTD ? pix_count : pix_count * sample_count;
+}
+
 // Runs one fused pass over the given work items (all with the same rng mode). Asynchronous on
 // ctx->stream; the caller synchronizes before reading results.
 int Context::run_pass(std::vector<WorkItem>& items, bool time_stages, double* extend_ms, const PassBufs& B) {
@@ -756,6 +779,57 @@ int Context::run_pass(std::vector<WorkItem>& items, bool time_stages, double* ex
     return CRT_OK;
 }
 
+// Runs one pass of whole-path launches: every work item (one request) is one launch that traces and
+// shades its paths to their end, and its resolve. The launches go round the sub-pass streams, so the
+// last paths of one request overlap the next one's. Asynchronous like run_pass.
+int Context::run_whole(std::vector<WorkItem>& items, const PassBufs& B) {
+    const int buf = pass_parity;
+    pass_parity ^= 1;
+    HIP_TRY(hipEventSynchronize(req_event[buf]));
+    crt_dev_request* host = (crt_dev_request*)req_host[buf];
+    uint32_t base = 0;
+    for (size_t k = 0; k < items.size(); ++k) {
+        const WorkItem& w = items[k];
+        crt_dev_request r = w.job->req;
+        r.path_base = base;
+        r.pix_begin = w.pix_begin; r.pix_count = w.pix_count;
+        r.sample_begin = w.sample_begin; r.sample_count = w.sample_count;
+        host[k] = r;
+        base += w.whole_ids();
+        w.job->rays_in_flight += (uint64_t)w.pix_count * w.sample_count;
+    }
+    if (base > B.pass_ids) return set_error(CRT_ERR_INTERNAL, "pass exceeds the pass capacity");
+    crt_dev_request* dreq = B.req[buf];
+    HIP_TRY(hipMemcpyAsync(dreq, host, sizeof(crt_dev_request) * items.size(), hipMemcpyHostToDevice, stream));
+    if (crt_k_fill_u32(stream, B.next, (uint32_t)items.size(), 0u)) return set_error(CRT_ERR_HIP, "fill launch failed");
+    const uint32_t K = (uint32_t)std::min<size_t>(items.size(), std::min(sub_passes, B.max_sub));
+    if (K > 1) HIP_TRY(hipEventRecord(ev_pass_ready, stream));
+    for (uint32_t q = 1; q < K; ++q) HIP_TRY(hipStreamWaitEvent(sub_stream[q - 1], ev_pass_ready, 0));
+    // overflow stacks: an equal share of the allocation for each stream
+    const uint64_t wave_words = 64ull * crt_k_paths_overflow_entries();
+    const uint64_t waves = B.gstack_words / K / wave_words;
+    if (waves == 0) return set_error(CRT_ERR_INTERNAL, "traversal stacks too small");
+    for (size_t k = 0; k < items.size(); ++k) {
+        const WorkItem& w = items[k];
+        const uint32_t q = (uint32_t)(k % K);
+        hipStream_t s = q == 0 ? stream : sub_stream[q - 1];
+        const HostScene& H = w.job->scene->host;
+        if (crt_k_paths(s, (int)w.job->rd.rng_mode, H.num_instances ? 1 : 0, H.num_shapes ? 1 : 0,
+                        (uint32_t)std::min<uint64_t>(waves, 1u << 20), (const crt_dev_scene*)scene_table.p, dreq + k,
+                        w.whole_ids(), B.next + k, B.out_rad + host[k].path_base, B.gstack + q * waves * wave_words, B.counters))
+            return set_error(CRT_ERR_HIP, "path launch failed");
+        if (w.job->rd.rng_mode == CRT_RNG_PCG && crt_k_resolve(s, dreq + k, 1, w.pix_count, B.out_rad, nullptr))
+            return set_error(CRT_ERR_HIP, "resolve launch failed");
+    }
+    for (uint32_t q = 1; q < K; ++q) {
+        HIP_TRY(hipEventRecord(sub_done[q - 1], sub_stream[q - 1]));
+        HIP_TRY(hipStreamWaitEvent(stream, sub_done[q - 1], 0));
+    }
+    HIP_TRY(hipEventRecord(req_event[buf], stream));
+    passes++;
+    return CRT_OK;
+}
+
 // One megakernel launch over the whole request (every pixel, every remaining sample in order).
 int Context::run_plain(Job& j, bool time_stages, double* extend_ms) {
     if (j.scheduled_all()) return CRT_OK;
@@ -842,6 +916,26 @@ int Context::render_jobs(std::vector<Job*>& jobs, bool time_stages, crt_stats* s
         if (!(j->rd.flags & CRT_RENDER_MEGAKERNEL)) continue;
         paths += (uint64_t)j->npix * (j->s_end - j->s_next);
         if ((rc = run_plain(*j, time_stages, &ext_ms))) return rc;
+    }
+    // Whole-path launches, unless the caller asked for the stages: timed or counted, or with one of
+    // the closest-hit stage's own work distributions. Scenes with two-wide nodes run in stages.
+    auto whole = [&](const Job* j) {
+        return !staged && !time_stages && j->scene->host.bvh_width == 4 && !(j->rd.flags & CRT_RENDER_MEGAKERNEL) && !j->scheduled_all();
+    };
+    for (;;) {
+        std::vector<WorkItem> items;
+        // the launch's hand-out counter runs past the last id by the chunks of its waves
+        uint32_t cap = std::min(B.pass_ids, 1u << 31);
+        for (Job* j : jobs) {
+            WorkItem w;
+            if (cap == 0 || items.size() >= B.max_requests) break;
+            if (!whole(j) || !j->take_whole(cap, w)) continue;
+            cap -= w.whole_ids();
+            paths += (uint64_t)w.pix_count * w.sample_count;
+            items.push_back(w);
+        }
+        if (items.empty()) break;
+        if ((rc = run_whole(items, B))) return rc;
     }
     // Passes of one scene run the single-scene traversal kernel and keep one tree in the caches.
     // A request with at least batch_group path ids left leads a pass of its own scene (with every

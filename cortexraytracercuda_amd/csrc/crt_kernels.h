@@ -49,6 +49,13 @@ int crt_k_shade(hipStream_t s, int rng_mode, int full, uint32_t grid, const crt_
                 crt_dev_counters* counters);
 int crt_k_plain(hipStream_t s, int rng_mode, int width, int two_level, uint32_t grid, const crt_dev_scene* scenes,
                 const crt_dev_request* req, uint32_t* gstack, crt_dev_counters* counters);
+// Whole paths of one request in one launch (paths.hip). `total` ids (pixels x samples, or pixels for
+// MINSTD, whose samples run in turn); `next` zeroed; `out_rad` at the request's first id; `gstack` room
+// for max_waves * 64 * crt_k_paths_overflow_entries() words.
+uint32_t crt_k_paths_overflow_entries(void);
+int crt_k_paths(hipStream_t s, int rng_mode, int two_level, int shapes, uint32_t max_waves, const crt_dev_scene* scenes,
+                const crt_dev_request* req, uint32_t total, uint32_t* next, float4* out_rad, uint32_t* gstack,
+                crt_dev_counters* counters);
 int crt_k_trace_rays(hipStream_t s, int width, int two_level, uint32_t grid, const crt_dev_scene* sc, const float4* rays, uint32_t n, int camera,
                      float4* hit, uint32_t* hit_inst, uint32_t* gstack, crt_dev_counters* counters);
 // rays (nreq == 1 only, may be null): the closest-hit queries of the resolved paths are added to it

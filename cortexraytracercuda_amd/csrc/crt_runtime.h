@@ -75,6 +75,7 @@ struct PassBufs {
     float4* hit; uint32_t* hit_inst;
     float4* out_rad;                // 16 B per path id of a pass
     uint32_t* gstack;               // traversal overflow stacks of extend_grid workgroups
+    uint64_t gstack_words;          // their 32-bit words
     uint32_t* ctl;                  // 2 * CRT_CTL_WORDS words per sub-pass
     crt_dev_counters* counters;
     crt_dev_request* req[2];        // device request tables (alternating between passes)
@@ -82,6 +83,8 @@ struct PassBufs {
     uint32_t pass_ids;              // path ids per pass
     uint32_t extend_grid;           // closest-hit workgroups
     uint32_t max_sub;               // concurrent sub-passes the buffers allow
+    uint32_t* next;                 // path hand-out counters of whole-path launches, one per request of a pass
+    uint32_t max_requests;          // requests of a pass
     crt_paths paths(int k, uint32_t slot0) const {
         crt_paths p;
         p.ray_o = ray_o[k] + slot0; p.ray_d = ray_d[k] + slot0; p.thr = thr[k] + slot0; p.rad = rad[k] + slot0;
@@ -94,6 +97,8 @@ struct Job;
 struct WorkItem {
     Job* job = nullptr;
     uint32_t pix_begin = 0, pix_count = 0, sample_begin = 0, sample_count = 0;
+    // path ids of a whole-path launch (a MINSTD pixel's samples run one after the other in one id)
+    uint32_t whole_ids() const;
 };
 
 struct Job {
@@ -113,6 +118,8 @@ struct Job {
     // a job whose accumulation buffer the caller owns (device memory): no allocation
     void setup_external(DeviceScene* sc, const crt_render_desc& r, float* accum_dev);
     bool take(uint32_t cap, WorkItem& w);
+    // the same for a whole-path launch: a MINSTD job gives pixels with all of their samples
+    bool take_whole(uint32_t cap, WorkItem& w);
     bool scheduled_all() const { return s_next >= s_end; }
     // path ids not yet handed to a pass
     uint64_t paths_left() const { return s_next >= s_end ? 0 : (uint64_t)(s_end - s_next) * npix - p_next; }
@@ -198,6 +205,7 @@ struct Context {
     int extend_mode = CRT_EXTEND_GRID_STRIDE;   // closest-hit work distribution (CRT_EXTEND_*)
     uint32_t extend_param = 2;       // lane-refill threshold or 64-ray groups per wave fetch
     uint32_t stack_lds = 16;         // LDS ring entries per lane of the traversal stack (8, 16, 32)
+    bool staged = false;             // blocking renders run as stage launches (asked for by extend_kernel, ray_sort or count_work)
     uint32_t ray_sort = 0;           // shade groups each block's survivors by direction octant
     uint32_t bvh_builder = CRT_BVH_HOST;   // where crt_scene_upload builds the BVH (CRT_BVH_*)
     uint64_t batch_group = 1ull << 22;     // path ids left for a batched request to get passes of its own scene
@@ -213,7 +221,7 @@ struct Context {
     std::map<crt_scene_id, std::unique_ptr<DeviceScene>> scenes;
     bool slot_used[kMaxScenes] = {};
     crt_scene_id next_scene_id = 1;
-    DevBuf scene_table, counters, ctl, gstack;
+    DevBuf scene_table, counters, ctl, gstack, path_next;
     DevBuf req_table[2];
     void* req_host[2] = {nullptr, nullptr};
     hipEvent_t req_event[2] = {nullptr, nullptr};
@@ -282,6 +290,7 @@ struct Context {
     DeviceScene* find_scene(crt_scene_id id);
     PassBufs pool_bufs();
     int run_pass(std::vector<WorkItem>& items, bool time_stages, double* extend_ms, const PassBufs& B);
+    int run_whole(std::vector<WorkItem>& items, const PassBufs& B);
     int run_plain(Job& j, bool time_stages, double* extend_ms);
     int finish_job(Job& j, crt_image* out);
     int reset_counters(crt_dev_counters* c);

@@ -120,6 +120,9 @@ int Context::autotune(crt_scene_id scene, const crt_scene_desc* desc, const crt_
         sc = find_scene(scene);
     }
 
+    // whole-path launches (four-wide scenes) have one tunable, their streams; the others belong to the stages
+    const bool stages = staged || sc->host.bvh_width != 4;
+
     // launch and memory shape, one tunable at a time
     Shape bs = current_shape(*this);
     auto apply = [&](const Shape& s) -> int {
@@ -160,20 +163,20 @@ int Context::autotune(crt_scene_id scene, const crt_scene_desc* desc, const crt_
         }
         return apply(bs);
     };
-    if ((rc = sweep([](Shape& s, uint32_t v) { s.slots = v; }, {1u << 23, 1u << 24, 1u << 25, 1u << 26}))) return rc;
-    if ((rc = sweep([](Shape& s, uint32_t v) { s.grid = v; }, {12u, 24u, 32u}))) return rc;
-    if ((rc = sweep([](Shape& s, uint32_t v) { s.sgrid = v; }, {4u, 8u, 16u}))) return rc;
+    if (stages && (rc = sweep([](Shape& s, uint32_t v) { s.slots = v; }, {1u << 23, 1u << 24, 1u << 25, 1u << 26}))) return rc;
+    if (stages && (rc = sweep([](Shape& s, uint32_t v) { s.grid = v; }, {12u, 24u, 32u}))) return rc;
+    if (stages && (rc = sweep([](Shape& s, uint32_t v) { s.sgrid = v; }, {4u, 8u, 16u}))) return rc;
     if ((rc = sweep([](Shape& s, uint32_t v) { s.sub = v; }, {1u, 2u, 3u, 4u}))) return rc;
     // closest-hit work distribution: grid-stride (coherent waves) or per-lane refill from the
     // wave's share of the queue after 16 / 32 idle lanes (fewer idle lanes on long, uneven rays)
-    if ((rc = sweep(
+    if (stages && (rc = sweep(
              [](Shape& s, uint32_t v) {
                  s.mode = v == 0 ? (uint32_t)CRT_EXTEND_GRID_STRIDE : (uint32_t)CRT_EXTEND_PERSISTENT;
                  s.param = v == 0 ? 2u : v;
              },
              {0u, 16u, 32u})))
         return rc;
-    if ((rc = sweep([](Shape& s, uint32_t v) { s.lds = v; }, {8u, 16u, 32u}))) return rc;
+    if (stages && (rc = sweep([](Shape& s, uint32_t v) { s.lds = v; }, {8u, 16u, 32u}))) return rc;
 
     out->max_paths = max_paths;
     out->grid_per_cu = grid_per_cu;
