@@ -105,7 +105,7 @@ template <class T> static int upload_vec(DevBuf& b, const std::vector<T>& v, Con
     if (v.empty()) { b.release(); return CRT_OK; }
     int rc = b.alloc(v.size() * sizeof(T), ctx);
     if (rc) return rc;
-    HIP_TRY(hipMemcpyAsync(b.p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice, s));
+    HIP_TRY(ctx->stage.push(b.p, v.data(), v.size() * sizeof(T), s));
     return CRT_OK;
 }
 
@@ -210,7 +210,7 @@ int Context::init(const crt_config* cfg) {
         HIP_TRY(hipHostMalloc(&req_host[k], sizeof(crt_dev_request) * kMaxPassRequests, hipHostMallocDefault));
         HIP_TRY(hipEventCreateWithFlags(&req_event[k], hipEventDisableTiming));
     }
-    HIP_TRY(hipHostMalloc((void**)&counters_host, sizeof(crt_dev_counters), hipHostMallocDefault));
+    if ((rc = stage.init(device))) return rc;
     HIP_TRY(hipEventCreate(&ev_start));
     HIP_TRY(hipEventCreate(&ev_stop));
     HIP_TRY(hipEventCreate(&ev_ext[0]));
@@ -336,7 +336,6 @@ Context::~Context() {
         if (req_host[k]) (void)hipHostFree(req_host[k]);
         if (req_event[k]) (void)hipEventDestroy(req_event[k]);
     }
-    if (counters_host) (void)hipHostFree(counters_host);
     for (int k = 0; k < kMaxSubPasses - 1; ++k) if (sub_stream[k]) (void)hipStreamSynchronize(sub_stream[k]);
     if (ctl_host) (void)hipHostFree(ctl_host);
     for (int k = 0; k < kCtlRing * kMaxSubPasses; ++k) if (ctl_ev[k]) (void)hipEventDestroy(ctl_ev[k]);
@@ -429,7 +428,7 @@ int Context::upload_scene_locked(const crt_scene_desc* desc, uint32_t leaf, uint
                                    {H.quads.data(), H.quads.size() * sizeof(F4), (size_t)H.quad_offset()}};
             if ((rc = sc->geo.alloc((size_t)H.geometry_bytes() + 256, this))) return rc;
             for (const Part& q : parts)
-                if (q.bytes) HIP_TRY(hipMemcpyAsync((char*)sc->geo.p + q.off, q.src, q.bytes, hipMemcpyHostToDevice, stream));
+                HIP_TRY(stage.push((char*)sc->geo.p + q.off, q.src, q.bytes, stream));
         }
         if ((rc = upload_vec(sc->tri_normals, H.tri_normals, this, stream))) return rc;
         if ((rc = upload_vec(sc->tri_uvs, H.tri_uvs, this, stream))) return rc;
@@ -451,7 +450,7 @@ int Context::upload_scene_locked(const crt_scene_desc* desc, uint32_t leaf, uint
         H.num_node_records = H.nodes.size() / (H.bvh_width == 4 ? 8u : 4u);
         H.num_tri_records = H.tris.size() / 3;
     }
-    HIP_TRY(hipMemcpyAsync((crt_dev_scene*)scene_table.p + slot, &sc->dev, sizeof(crt_dev_scene), hipMemcpyHostToDevice, stream));
+    HIP_TRY(stage.push((crt_dev_scene*)scene_table.p + slot, &sc->dev, sizeof(crt_dev_scene), stream));
     HIP_TRY(hipStreamSynchronize(stream));
     sc->upload_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
     sc->slot = slot;
@@ -491,7 +490,8 @@ int Context::verify_scene(const DeviceScene& sc, std::string& err) {
     V.quads.resize(nq * 5);
     V.insts.resize(sc.inst_gid.size() * 4);
     auto rd = [&](std::vector<F4>& v, const void* src) -> int {
-        if (!v.empty()) HIP_TRY(hipMemcpyAsync(v.data(), src, v.size() * sizeof(F4), hipMemcpyDeviceToHost, stream));
+        const HostStage::Copy c{v.data(), src, v.size() * sizeof(F4)};
+        HIP_TRY(stage.fetch(&c, 1, stream));
         return CRT_OK;
     };
     int rc;
@@ -867,24 +867,9 @@ int Context::run_plain(Job& j, bool time_stages, double* extend_ms) {
     return CRT_OK;
 }
 
-int Context::finish_job(Job& j, crt_image* out) {
-    if (crt_k_tonemap(stream, (const float4*)j.accum.p, j.npix, j.rd.spp, (uint8_t*)j.rgb.p))
-        return set_error(CRT_ERR_HIP, "tonemap launch failed");
-    if (out && out->rgb8) HIP_TRY(hipMemcpyAsync(out->rgb8, j.rgb.p, (size_t)j.npix * 3, hipMemcpyDeviceToHost, stream));
-    if (out && out->accum) HIP_TRY(hipMemcpyAsync(out->accum, j.accum.p, (size_t)j.npix * 16, hipMemcpyDeviceToHost, stream));
-    return CRT_OK;
-}
-
 int Context::reset_counters(crt_dev_counters* c) {
     if (crt_k_fill_u32(stream, (uint32_t*)c, sizeof(crt_dev_counters) / 4, 0u))
         return set_error(CRT_ERR_HIP, "fill launch failed");
-    return CRT_OK;
-}
-
-int Context::read_counters(crt_dev_counters& c, const crt_dev_counters* dev) {
-    HIP_TRY(hipMemcpyAsync(counters_host, dev, sizeof(crt_dev_counters), hipMemcpyDeviceToHost, stream));
-    HIP_TRY(hipStreamSynchronize(stream));
-    c = *(crt_dev_counters*)counters_host;
     return CRT_OK;
 }
 
@@ -904,7 +889,7 @@ void fill_stats(crt_stats* st, const crt_dev_counters& c, uint64_t paths, double
 }
 
 // Plain and batched rendering: all items are admitted at once, passes are packed greedily.
-int Context::render_jobs(std::vector<Job*>& jobs, bool time_stages, crt_stats* stats, const PassBufs& B) {
+int Context::render_jobs(std::vector<Job*>& jobs, bool time_stages, crt_stats* stats, const PassBufs& B, crt_batch_item* out) {
     double h0 = now_s();
     int rc;
     if ((rc = reset_counters(B.counters))) return rc;
@@ -969,11 +954,19 @@ int Context::render_jobs(std::vector<Job*>& jobs, bool time_stages, crt_stats* s
         }
     }
     HIP_TRY(hipEventRecord(ev_stop, stream));
-    HIP_TRY(hipEventSynchronize(ev_stop));
+    crt_dev_counters c;
+    std::vector<HostStage::Copy> back{{&c, B.counters, sizeof(c)}};
+    for (size_t k = 0; out && k < jobs.size(); ++k) {
+        Job& j = *jobs[k];
+        const crt_image& img = out[k].out;
+        if (crt_k_tonemap(stream, (const float4*)j.accum.p, j.npix, j.rd.spp, (uint8_t*)j.rgb.p))
+            return set_error(CRT_ERR_HIP, "tonemap launch failed");
+        if (img.rgb8) back.push_back({img.rgb8, j.rgb.p, (size_t)j.npix * 3});
+        if (img.accum) back.push_back({img.accum, j.accum.p, (size_t)j.npix * 16});
+    }
+    HIP_TRY(stage.fetch(back.data(), (int)back.size(), stream));
     float gms = 0.0f;
     HIP_TRY(hipEventElapsedTime(&gms, ev_start, ev_stop));
-    crt_dev_counters c;
-    if ((rc = read_counters(c, B.counters))) return rc;
     if (c.stack_overflow) return set_error(CRT_ERR_INTERNAL, "traversal stack overflow");
     fill_stats(stats, c, paths, gms, ext_ms, (now_s() - h0) * 1e3);
     last.rays = c.rays + c.retraces; last.retraces = c.retraces; last.light_pdf_tests = c.light_tests;
@@ -1136,13 +1129,7 @@ int crt_render_batch(crt_context* c, crt_batch_item* items, uint32_t n, crt_stat
         jobs.push_back(std::move(j));
     }
     bool time_stages = (n > 0) && (items[0].rd.flags & CRT_RENDER_TIME_STAGES);
-    int rc = ctx->render_jobs(jp, time_stages, stats, ctx->pool_bufs());
-    if (rc) return rc;
-    for (uint32_t k = 0; k < n; ++k) {
-        if ((rc = ctx->finish_job(*jobs[k], &items[k].out))) return rc;
-    }
-    if (hipStreamSynchronize(ctx->stream) != hipSuccess) return set_error(CRT_ERR_HIP, "stream synchronize failed");
-    return CRT_OK;
+    return ctx->render_jobs(jp, time_stages, stats, ctx->pool_bufs(), items);
 }
 
 int crt_trace_rays(crt_context* c, crt_scene_id s, const float* rays, uint64_t n, int32_t flags, int32_t* prim,
@@ -1176,8 +1163,8 @@ int crt_trace_rays(crt_context* c, crt_scene_id s, const float* rays, uint64_t n
             po[4 * k + 3] = 0.0f;
             std::memcpy(&pd[4 * k + 3], &state, 4);
         }
-        HIP_TRY(hipMemcpyAsync(dro.p, po.data(), n * 16, hipMemcpyHostToDevice, ctx->stream));
-        HIP_TRY(hipMemcpyAsync(drd.p, pd.data(), n * 16, hipMemcpyHostToDevice, ctx->stream));
+        HIP_TRY(ctx->stage.push(dro.p, po.data(), n * 16, ctx->stream));
+        HIP_TRY(ctx->stage.push(drd.p, pd.data(), n * 16, ctx->stream));
         HIP_TRY(hipMemsetAsync(dids.p, 0, n * 8, ctx->stream));
         HIP_TRY(hipMemsetAsync(dctl.p, 0, CRT_CTL_WORDS * 4, ctx->stream));
         uint32_t* ctl = (uint32_t*)dctl.p;
@@ -1190,7 +1177,7 @@ int crt_trace_rays(crt_context* c, crt_scene_id s, const float* rays, uint64_t n
         HIP_TRY(hipStreamSynchronize(ctx->stream));
     } else {
         if ((rc = dr.alloc(n * 32, ctx))) return rc;
-        HIP_TRY(hipMemcpyAsync(dr.p, rays, n * 32, hipMemcpyHostToDevice, ctx->stream));
+        HIP_TRY(ctx->stage.push(dr.p, rays, n * 32, ctx->stream));
         if (crt_k_trace_rays(ctx->stream, (int)sc->host.bvh_width, two_level, grid,
                              (const crt_dev_scene*)ctx->scene_table.p + sc->slot, (const float4*)dr.p,
                              (uint32_t)n, camera ? 1 : 0, (float4*)dh.p, (uint32_t*)di.p, (uint32_t*)ctx->gstack.p,
@@ -1199,11 +1186,9 @@ int crt_trace_rays(crt_context* c, crt_scene_id s, const float* rays, uint64_t n
     }
     std::vector<float> hh(n * 4);
     std::vector<uint32_t> hi(n);
-    HIP_TRY(hipMemcpyAsync(hh.data(), dh.p, n * 16, hipMemcpyDeviceToHost, ctx->stream));
-    HIP_TRY(hipMemcpyAsync(hi.data(), di.p, n * 4, hipMemcpyDeviceToHost, ctx->stream));
-    HIP_TRY(hipStreamSynchronize(ctx->stream));
     crt_dev_counters cnt;
-    if ((rc = ctx->read_counters(cnt, (const crt_dev_counters*)ctx->counters.p))) return rc;
+    const HostStage::Copy back[3] = {{&cnt, ctx->counters.p, sizeof(cnt)}, {hh.data(), dh.p, n * 16}, {hi.data(), di.p, n * 4}};
+    HIP_TRY(ctx->stage.fetch(back, 3, ctx->stream));
     if (cnt.stack_overflow) return set_error(CRT_ERR_INTERNAL, "traversal stack overflow");
     // map leaf-ordered hits back to global ids: copies of the id words are kept on the host
     const HostScene& H = sc->host;

@@ -469,7 +469,7 @@ int gpu_build_scene(Context& C, const crt_scene_desc* d, uint32_t leaf, uint32_t
         if (!bytes) return CRT_OK;
         int r = b.alloc(bytes, ctx);
         if (r) return r;
-        HIP_TRY(hipMemcpyAsync(b.p, h, bytes, hipMemcpyHostToDevice, s));
+        HIP_TRY(ctx->stage.push(b.p, h, bytes, s));
         return CRT_OK;
     };
     if ((rc = up(squads, src.quads.data(), src.quads.size() * sizeof(F4)))) return rc;
@@ -609,16 +609,17 @@ int gpu_build_scene(Context& C, const crt_scene_desc* d, uint32_t leaf, uint32_t
                                  dptr<float4>(sc.tri_normals), dptr<float2>(sc.tri_uvs), dptr<float2>(sc.sphere_map),
                                  src_tri, src_sph, src_quad), "scatter");
     std::vector<uint32_t> srch((size_t)nt + ns + nq);
-    if (!srch.empty()) HIP_TRY(hipMemcpyAsync(srch.data(), srcmap.p, srch.size() * 4, hipMemcpyDeviceToHost, s));
+    const HostStage::Copy back{srch.data(), srcmap.p, srch.size() * 4};
+    HIP_TRY(ctx->stage.fetch(&back, 1, s));
     if ((rc = (sc.mats.alloc(H.mats.size() * 16, ctx)))) return rc;
-    if (!H.mats.empty()) HIP_TRY(hipMemcpyAsync(sc.mats.p, H.mats.data(), H.mats.size() * 16, hipMemcpyHostToDevice, s));
+    if (!H.mats.empty()) HIP_TRY(ctx->stage.push(sc.mats.p, H.mats.data(), H.mats.size() * 16, s));
     if (!H.texs.empty()) {
         if ((rc = sc.texs.alloc(H.texs.size() * 16, ctx))) return rc;
-        HIP_TRY(hipMemcpyAsync(sc.texs.p, H.texs.data(), H.texs.size() * 16, hipMemcpyHostToDevice, s));
+        HIP_TRY(ctx->stage.push(sc.texs.p, H.texs.data(), H.texs.size() * 16, s));
     }
     if (!H.texels.empty()) {
         if ((rc = sc.texels.alloc(H.texels.size(), ctx))) return rc;
-        HIP_TRY(hipMemcpyAsync(sc.texels.p, H.texels.data(), H.texels.size(), hipMemcpyHostToDevice, s));
+        HIP_TRY(ctx->stage.push(sc.texels.p, H.texels.data(), H.texels.size(), s));
     }
     HIP_TRY(hipStreamSynchronize(s));
     // host maps: leaf order -> global id
@@ -639,7 +640,7 @@ int gpu_build_scene(Context& C, const crt_scene_desc* d, uint32_t leaf, uint32_t
             table[i] = (s0 & CRT_LIGHT_SPHERE) ? (CRT_LIGHT_SPHERE | sph_slot[s0 & ~CRT_LIGHT_SPHERE]) : quad_slot[s0];
         }
         if ((rc = sc.lights.alloc(table.size() * 4, ctx))) return rc;
-        HIP_TRY(hipMemcpyAsync(sc.lights.p, table.data(), table.size() * 4, hipMemcpyHostToDevice, s));
+        HIP_TRY(ctx->stage.push(sc.lights.p, table.data(), table.size() * 4, s));
         HIP_TRY(hipStreamSynchronize(s));
     }
     // device scene record

@@ -16,6 +16,7 @@
 #include "cortex_rt.h"
 #include "crt_kernels.h"
 #include "crt_layout.h"
+#include "host_stage.h"
 #include "scene_build.h"
 
 namespace crt {
@@ -170,7 +171,6 @@ struct Server {
     crt_dev_request* req_host = nullptr;   // pinned mirror of the open pass's request table
     uint32_t* open_host = nullptr;         // pinned ring of (total, nreq)
     uint32_t* snap = nullptr;              // pinned ring of iteration snapshots
-    void* rays_host = nullptr;             // pinned word for a finished request's ray count
     hipEvent_t ev[kRing] = {};
     // open pass (host view)
     std::vector<SrvEntry> entries;
@@ -226,7 +226,8 @@ struct Context {
     void* req_host[2] = {nullptr, nullptr};
     hipEvent_t req_event[2] = {nullptr, nullptr};
     hipEvent_t ev_start = nullptr, ev_stop = nullptr, ev_ext[2] = {nullptr, nullptr};
-    void* counters_host = nullptr;
+    HostStage stage;                 // blocking calls' copies to and from the caller's memory (exec_mutex)
+    HostStage srv_stage;             // the completion thread's
     int pass_parity = 0;
     uint64_t passes = 0, extend_launches = 0, iterations = 0;
     // streaming pass: two compact path-state buffers of max_paths slots (alternating between
@@ -292,10 +293,9 @@ struct Context {
     int run_pass(std::vector<WorkItem>& items, bool time_stages, double* extend_ms, const PassBufs& B);
     int run_whole(std::vector<WorkItem>& items, const PassBufs& B);
     int run_plain(Job& j, bool time_stages, double* extend_ms);
-    int finish_job(Job& j, crt_image* out);
     int reset_counters(crt_dev_counters* c);
-    int read_counters(crt_dev_counters& c, const crt_dev_counters* dev);
-    int render_jobs(std::vector<Job*>& jobs, bool time_stages, crt_stats* stats, const PassBufs& B);
+    // `out`: the jobs' images (tonemapped and read back with the counters, one wait for all), or null
+    int render_jobs(std::vector<Job*>& jobs, bool time_stages, crt_stats* stats, const PassBufs& B, crt_batch_item* out = nullptr);
     // no-allocation render (crt_render_noalloc): passes run on the device's scratch array
     void* scratch = nullptr;         // this device's scratch array (hipGetSymbolAddress at init)
     size_t scratch_bytes = 0;

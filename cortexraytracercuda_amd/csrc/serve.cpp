@@ -126,7 +126,7 @@ int Context::server_init_lane(Server& S, uint32_t slots, uint32_t cap, bool firs
     HIP_TRY(hipHostMalloc((void**)&S.req_host, sizeof(crt_dev_request) * Server::kEntries, hipHostMallocDefault));
     HIP_TRY(hipHostMalloc((void**)&S.open_host, sizeof(uint32_t) * 2 * Server::kOpenRing, hipHostMallocDefault));
     HIP_TRY(hipHostMalloc((void**)&S.snap, sizeof(uint32_t) * Server::kSnapWords * Server::kRing, hipHostMallocDefault));
-    if (first) HIP_TRY(hipHostMalloc(&S.rays_host, sizeof(unsigned long long), hipHostMallocDefault));
+    if (first && (rc = srv_stage.init(device))) return rc;
     for (int k = 0; k < Server::kRing; ++k) HIP_TRY(hipEventCreateWithFlags(&S.ev[k], hipEventDisableTiming));
     if (crt_k_fill_u32(S.s, (uint32_t*)S.counters.p, sizeof(crt_dev_counters) / 4, 0u))
         return set_error(CRT_ERR_HIP, "fill launch failed");
@@ -158,14 +158,13 @@ void Context::server_release_lane(Server& S) {
     if (S.req_host) (void)hipHostFree(S.req_host);
     if (S.open_host) (void)hipHostFree(S.open_host);
     if (S.snap) (void)hipHostFree(S.snap);
-    if (S.rays_host) (void)hipHostFree(S.rays_host);
     for (int k = 0; k < Server::kRing; ++k) if (S.ev[k]) (void)hipEventDestroy(S.ev[k]);
     for (int t = 0; t < Server::kVariants; ++t)
         for (int k = 0; k < Server::kRing; ++k)
             if (S.graph[t][k]) { (void)hipGraphExecDestroy(S.graph[t][k]); S.graph[t][k] = nullptr; }
     if (S.s) (void)hipStreamDestroy(S.s);
     if (S.copy_s) (void)hipStreamDestroy(S.copy_s);
-    S.req_host = nullptr; S.open_host = nullptr; S.snap = nullptr; S.rays_host = nullptr; S.s = nullptr; S.copy_s = nullptr;
+    S.req_host = nullptr; S.open_host = nullptr; S.snap = nullptr; S.s = nullptr; S.copy_s = nullptr;
     S.ready = false;
 }
 
@@ -434,21 +433,20 @@ int Context::server_process_snapshot(Server& S, std::vector<ServeReq*>& act) {
 
 // Readback and completion of one finished request (completion thread; status != CRT_OK: no copies).
 void Context::server_complete(ServeReq* r, int st) {
-    Server& S = srv[0];   // owns the copy stream and the pinned ray-count word
+    Server& S = srv[0];   // owns the copy stream
     if (st == CRT_OK) {
         // the accumulation buffer (16 B per pixel against 3 for the image) only when asked for
         const bool want_accum = !(r->rd.flags & CRT_RENDER_IMAGE_ONLY);
         r->rgb.resize((size_t)r->job->npix * 3);
         r->accum.resize(want_accum ? (size_t)r->job->npix * 4 : 0);
-        unsigned long long* rays_h = (unsigned long long*)S.rays_host;
-        if (hipMemcpyAsync(rays_h, r->job->rays_counter(), sizeof(*rays_h), hipMemcpyDeviceToHost, S.copy_s) != hipSuccess ||
-            hipMemcpyAsync(r->rgb.data(), r->job->rgb.p, r->rgb.size(), hipMemcpyDeviceToHost, S.copy_s) != hipSuccess ||
-            (want_accum && hipMemcpyAsync(r->accum.data(), r->job->accum.p, r->accum.size() * sizeof(float),
-                                          hipMemcpyDeviceToHost, S.copy_s) != hipSuccess) ||
-            hipStreamSynchronize(S.copy_s) != hipSuccess)
+        unsigned long long rays = 0;
+        const HostStage::Copy back[3] = {{&rays, r->job->rays_counter(), sizeof(rays)},
+                                         {r->rgb.data(), r->job->rgb.p, r->rgb.size()},
+                                         {r->accum.data(), r->job->accum.p, r->accum.size() * sizeof(float)}};
+        if (srv_stage.fetch(back, 3, S.copy_s) != hipSuccess)
             st = set_error(CRT_ERR_HIP, "readback failed");
         else
-            r->timing.rays = *rays_h;
+            r->timing.rays = rays;
     }
     if (r->ev_done) { (void)hipEventDestroy(r->ev_done); r->ev_done = nullptr; }
     // the job's buffers go back to the cache (own lock); its stream work has completed
