@@ -1141,22 +1141,27 @@ int crt_trace_rays(crt_context* c, crt_scene_id s, const float* rays, uint64_t n
     DeviceScene* sc = ctx->find_scene(s);
     if (!sc) return set_error(CRT_ERR_INVALID_ARGUMENT, "unknown scene id");
     if (n == 0) return CRT_OK;
-    DevBuf dr, dh, di;
+    // per-call buffers from the context's cache; large ones at their own size (the cache's classes are
+    // powers of two)
+    auto get = [&](DevBuf& b, uint64_t bytes) { return bytes <= (256ull << 20) ? b.alloc_cached(bytes, ctx) : b.alloc(bytes, ctx); };
+    DevBuf out;
     int rc;
     const bool camera = (flags & CRT_TRACE_CAMERA) != 0;
-    if ((rc = dh.alloc(n * 16, ctx))) return rc;
-    if ((rc = di.alloc(n * 4, ctx))) return rc;
+    if ((rc = get(out, n * 20))) return rc;
     if ((rc = ctx->reset_counters((crt_dev_counters*)ctx->counters.p))) return rc;
     uint32_t grid = std::min(ctx->extend_grid, (uint32_t)std::max<uint64_t>(1, (n + 255) / 256));
     const int two_level = sc->host.num_instances ? (sc->host.num_shapes ? 2 : 1) : 0;
+    const crt_dev_scene* dsc = (const crt_dev_scene*)ctx->scene_table.p;
+    DevBuf dr, dh, di, dro, drd, dids, dctl;   // until the results are here
+    std::vector<float> po, pd;
     if (flags & CRT_TRACE_STAGE) {
         // the render's closest-hit stage: path-state rays (origin, time 0; direction, depth 1 and the
         // camera bit), one uniform scene, the stage's control words
-        DevBuf dro, drd, dids, dctl;
-        if ((rc = dro.alloc(n * 16, ctx)) || (rc = drd.alloc(n * 16, ctx)) || (rc = dids.alloc(n * 8, ctx)) ||
-            (rc = dctl.alloc(CRT_CTL_WORDS * 4, ctx)))
+        if ((rc = get(dh, n * 16)) || (rc = get(di, n * 4)) || (rc = get(dro, n * 16)) || (rc = get(drd, n * 16)) ||
+            (rc = get(dids, n * 8)) || (rc = get(dctl, CRT_CTL_WORDS * 4)))
             return rc;
-        std::vector<float> po(n * 4), pd(n * 4);
+        po.resize(n * 4);
+        pd.resize(n * 4);
         const uint32_t state = 1u | (camera ? 0x10000u : 0u);   // depth 1 | camera bit of the path state
         for (uint64_t k = 0; k < n; ++k) {
             for (int a = 0; a < 3; ++a) { po[4 * k + a] = rays[8 * k + a]; pd[4 * k + a] = rays[8 * k + 4 + a]; }
@@ -1168,46 +1173,30 @@ int crt_trace_rays(crt_context* c, crt_scene_id s, const float* rays, uint64_t n
         HIP_TRY(hipMemsetAsync(dids.p, 0, n * 8, ctx->stream));
         HIP_TRY(hipMemsetAsync(dctl.p, 0, CRT_CTL_WORDS * 4, ctx->stream));
         uint32_t* ctl = (uint32_t*)dctl.p;
-        if (crt_k_extend(ctx->stream, ctx->config.count_work ? 1 : 0, (int)sc->host.bvh_width, two_level, grid,
-                         (const crt_dev_scene*)ctx->scene_table.p, nullptr, (int32_t)sc->slot, nullptr, nullptr,
-                         (uint32_t)n, (const float4*)dro.p, (const float4*)drd.p, (const uint2*)dids.p, (float4*)dh.p,
-                         (uint32_t*)di.p, (uint32_t*)ctx->gstack.p, nullptr, ctx->extend_mode, ctl + CRT_CTL_WORK,
-                         ctx->extend_param, (int)ctx->stack_lds, nullptr, (crt_dev_counters*)ctx->counters.p))
+        if (crt_k_extend(ctx->stream, ctx->config.count_work ? 1 : 0, (int)sc->host.bvh_width, two_level, grid, dsc, nullptr,
+                         (int32_t)sc->slot, nullptr, nullptr, (uint32_t)n, (const float4*)dro.p, (const float4*)drd.p,
+                         (const uint2*)dids.p, (float4*)dh.p, (uint32_t*)di.p, (uint32_t*)ctx->gstack.p, nullptr,
+                         ctx->extend_mode, ctl + CRT_CTL_WORK, ctx->extend_param, (int)ctx->stack_lds, nullptr,
+                         (crt_dev_counters*)ctx->counters.p))
             return set_error(CRT_ERR_HIP, "extend launch failed");
-        HIP_TRY(hipStreamSynchronize(ctx->stream));
+        if (crt_k_report_hits(ctx->stream, grid, dsc + sc->slot, (const float4*)dh.p, (const uint32_t*)di.p, (uint32_t)n,
+                              (uint32_t*)out.p))
+            return set_error(CRT_ERR_HIP, "report launch failed");
     } else {
-        if ((rc = dr.alloc(n * 32, ctx))) return rc;
+        if ((rc = get(dr, n * 32))) return rc;
         HIP_TRY(ctx->stage.push(dr.p, rays, n * 32, ctx->stream));
-        if (crt_k_trace_rays(ctx->stream, (int)sc->host.bvh_width, two_level, grid,
-                             (const crt_dev_scene*)ctx->scene_table.p + sc->slot, (const float4*)dr.p,
-                             (uint32_t)n, camera ? 1 : 0, (float4*)dh.p, (uint32_t*)di.p, (uint32_t*)ctx->gstack.p,
+        if (crt_k_trace_rays(ctx->stream, (int)sc->host.bvh_width, two_level, grid, dsc + sc->slot, (const float4*)dr.p,
+                             (uint32_t)n, camera ? 1 : 0, (uint32_t*)out.p, (uint32_t*)ctx->gstack.p,
                              (crt_dev_counters*)ctx->counters.p))
             return set_error(CRT_ERR_HIP, "trace launch failed");
     }
-    std::vector<float> hh(n * 4);
-    std::vector<uint32_t> hi(n);
     crt_dev_counters cnt;
-    const HostStage::Copy back[3] = {{&cnt, ctx->counters.p, sizeof(cnt)}, {hh.data(), dh.p, n * 16}, {hi.data(), di.p, n * 4}};
-    HIP_TRY(ctx->stage.fetch(back, 3, ctx->stream));
+    const char* o = (const char*)out.p;
+    const HostStage::Copy back[5] = {{&cnt, ctx->counters.p, sizeof(cnt)}, {prim, o, prim ? n * 4 : 0},
+                                     {inst, o + n * 4, inst ? n * 4 : 0}, {t, o + n * 8, t ? n * 4 : 0},
+                                     {uv, o + n * 12, uv ? n * 8 : 0}};
+    HIP_TRY(ctx->stage.fetch(back, 5, ctx->stream));
     if (cnt.stack_overflow) return set_error(CRT_ERR_INTERNAL, "traversal stack overflow");
-    // map leaf-ordered hits back to global ids: copies of the id words are kept on the host
-    const HostScene& H = sc->host;
-    for (uint64_t k = 0; k < n; ++k) {
-        uint32_t p;
-        std::memcpy(&p, &hh[4 * k + 1], 4);
-        int32_t gid = -1;
-        if (p != CRT_MISS) {
-            uint32_t type = CRT_HIT_TYPE(p), idx = CRT_HIT_INDEX(p);
-            if (type == CRT_PRIM_TRI) gid = (int32_t)sc->tri_gid[idx];
-            else if (type == CRT_PRIM_SPHERE) gid = (int32_t)H.sphere_aux[idx].x;
-            else gid = (int32_t)sc->quad_gid[idx];
-        }
-        if (prim) prim[k] = gid;
-        const uint32_t iw = hi[k] & CRT_INST_MASK;
-        if (inst) inst[k] = (p == CRT_MISS || iw == CRT_NO_INST) ? -1 : (int32_t)sc->inst_gid[iw];
-        if (t) t[k] = p == CRT_MISS ? 0.0f : hh[4 * k];
-        if (uv) { uv[2 * k] = p == CRT_MISS ? 0.0f : hh[4 * k + 2]; uv[2 * k + 1] = p == CRT_MISS ? 0.0f : hh[4 * k + 3]; }
-    }
     return CRT_OK;
 }
 

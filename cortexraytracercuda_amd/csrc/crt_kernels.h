@@ -56,8 +56,11 @@ uint32_t crt_k_paths_overflow_entries(void);
 int crt_k_paths(hipStream_t s, int rng_mode, int two_level, int shapes, uint32_t max_waves, const crt_dev_scene* scenes,
                 const crt_dev_request* req, uint32_t total, uint32_t* next, float4* out_rad, uint32_t* gstack,
                 crt_dev_counters* counters);
-int crt_k_trace_rays(hipStream_t s, int width, int two_level, uint32_t grid, const crt_dev_scene* sc, const float4* rays, uint32_t n, int camera,
-                     float4* hit, uint32_t* hit_inst, uint32_t* gstack, crt_dev_counters* counters);
+// Closest hits of n rays into `out`: n primitive ids, n instance ids, n distances, n (u, v) pairs.
+int crt_k_trace_rays(hipStream_t s, int width, int two_level, uint32_t grid, const crt_dev_scene* sc, const float4* rays,
+                     uint32_t n, int camera, uint32_t* out, uint32_t* gstack, crt_dev_counters* counters);
+int crt_k_report_hits(hipStream_t s, uint32_t grid, const crt_dev_scene* sc, const float4* hit, const uint32_t* hit_inst,
+                      uint32_t n, uint32_t* out);
 // rays (nreq == 1 only, may be null): the closest-hit queries of the resolved paths are added to it
 int crt_k_resolve(hipStream_t s, const crt_dev_request* reqs, int nreq, uint32_t max_pix, const float4* rad,
                   unsigned long long* rays);
