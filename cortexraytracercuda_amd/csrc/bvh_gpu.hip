@@ -8,7 +8,8 @@
 //   3. the binary radix tree over the sorted codes (Karras, "Maximizing parallelism in the
 //      construction of BVHs, octrees, and k-d trees", HPG 2012): one thread per internal node,
 //      equal codes ordered by position;
-//   4. boxes fitted bottom-up, one thread per leaf climbing while it is the second child to arrive;
+//   4. boxes of the nodes as range minima and maxima: a node covers a run of the sorted primitives, so
+//      a binary tree over the sorted positions answers it in at most two boxes a level;
 //   5. per-type ranks of the sorted primitives (exclusive scan): a leaf's records are a contiguous
 //      run of its type's array in sorted order, so a leaf reference is (type, first rank, count);
 //   6. a top-down pass per level turns the binary tree into the traversal's nodes: four-wide nodes
@@ -165,8 +166,7 @@ __device__ __forceinline__ int delta(const uint64_t* __restrict__ k, int n, int 
 // 3. binary radix tree: internal node i covers sorted positions [first, first + count); children
 // >= 0 are internal nodes, < 0 leaves (~position)
 __global__ __launch_bounds__(256) void k_bvh_karras(const uint64_t* __restrict__ k, int n, int32_t* __restrict__ cl,
-                                                    int32_t* __restrict__ cr, int32_t* __restrict__ parent,
-                                                    int32_t* __restrict__ leaf_parent, uint32_t* __restrict__ first,
+                                                    int32_t* __restrict__ cr, uint32_t* __restrict__ first,
                                                     uint32_t* __restrict__ count) {
     for (int i = blockIdx.x * 256 + threadIdx.x; i < n - 1; i += gridDim.x * 256) {
         const int d = (delta(k, n, i, i + 1) - delta(k, n, i, i - 1)) >= 0 ? 1 : -1;
@@ -188,47 +188,77 @@ __global__ __launch_bounds__(256) void k_bvh_karras(const uint64_t* __restrict__
         const int32_t left = lo == g ? ~g : g, right = hi == g + 1 ? ~(g + 1) : g + 1;
         cl[i] = left;
         cr[i] = right;
-        if (left < 0) leaf_parent[~left] = i; else parent[left] = i;
-        if (right < 0) leaf_parent[~right] = i; else parent[right] = i;
         first[i] = (uint32_t)lo;
         count[i] = (uint32_t)(hi - lo + 1);
-        if (i == 0) parent[0] = -1;
     }
 }
 
-// 4. boxes bottom-up: each leaf climbs; at every node the first of the two children to arrive stops,
-// the second fits the node's box (and its type mask) from both children and goes on
-__global__ __launch_bounds__(256) void k_bvh_refit(int n, const uint32_t* __restrict__ vals, const float4* __restrict__ plo,
-                                                   const float4* __restrict__ phi, const int32_t* __restrict__ cl,
-                                                   const int32_t* __restrict__ cr, const int32_t* __restrict__ parent,
-                                                   const int32_t* __restrict__ leaf_parent, float4* nlo, float4* nhi,
-                                                   uint32_t* tmask, uint32_t* __restrict__ visits) {
-    for (int s = blockIdx.x * 256 + threadIdx.x; s < n; s += gridDim.x * 256) {
-        int node = leaf_parent[s];
-        while (node >= 0) {
-            __threadfence();
-            if (atomicAdd(visits + node, 1u) == 0u) break;
-            __threadfence();
-            float4 lo[2], hi[2];
-            uint32_t tm = 0;
-            const int32_t ch[2] = {cl[node], cr[node]};
-            for (int c = 0; c < 2; ++c) {
-                if (ch[c] < 0) {
-                    const uint32_t p = vals[~ch[c]];
-                    lo[c] = plo[p]; hi[c] = phi[p];
-                    tm |= 1u << __float_as_uint(lo[c].w);
-                } else {
-                    // written by the thread that completed the child, before its fence and atomic
-                    lo[c] = nlo[ch[c]];
-                    hi[c] = nhi[ch[c]];
-                    tm |= tmask[ch[c]];
-                }
-            }
-            nlo[node] = make_float4(fminf(lo[0].x, lo[1].x), fminf(lo[0].y, lo[1].y), fminf(lo[0].z, lo[1].z), 0.0f);
-            nhi[node] = make_float4(fmaxf(hi[0].x, hi[1].x), fmaxf(hi[0].y, hi[1].y), fmaxf(hi[0].z, hi[1].z), 0.0f);
-            tmask[node] = tm;
-            node = parent[node];
+// 4. boxes. Level 0 of the range tree holds the boxes of the sorted primitives (type mask in lo.w),
+// level k the unions of pairs of level k - 1; all levels lie one behind the other.
+struct RangeLevels {
+    static constexpr int kMax = 32;
+    uint32_t at[kMax], size[kMax];   // first entry and entries of each level
+    int levels;
+};
+
+__device__ __forceinline__ void box_union(float4& lo, float4& hi, float4 l, float4 h) {
+    lo = make_float4(fminf(lo.x, l.x), fminf(lo.y, l.y), fminf(lo.z, l.z), __uint_as_float(__float_as_uint(lo.w) | __float_as_uint(l.w)));
+    hi = make_float4(fmaxf(hi.x, h.x), fmaxf(hi.y, h.y), fmaxf(hi.z, h.z), 0.0f);
+}
+
+// Eight levels above `base`: a workgroup unites 256 of its entries down to one in LDS. With base 0 it
+// first gathers the primitives' boxes into level 0.
+__global__ __launch_bounds__(256) void k_bvh_range(RangeLevels L, int base, const uint32_t* __restrict__ vals,
+                                                   const float4* __restrict__ plo, const float4* __restrict__ phi,
+                                                   float4* __restrict__ rlo, float4* __restrict__ rhi) {
+    __shared__ float4 slo[256], shi[256];
+    const uint32_t t = threadIdx.x, i = blockIdx.x * 256u + t, n = L.size[base];
+    const float inf = __builtin_inff();
+    float4 lo = make_float4(inf, inf, inf, 0.0f), hi = make_float4(-inf, -inf, -inf, 0.0f);
+    if (i < n) {
+        if (base == 0) {
+            const uint32_t p = vals[i];
+            lo = plo[p]; hi = phi[p];
+            lo.w = __uint_as_float(1u << __float_as_uint(lo.w));
+            rlo[i] = lo; rhi[i] = hi;
+        } else {
+            lo = rlo[L.at[base] + i]; hi = rhi[L.at[base] + i];
         }
+    }
+    slo[t] = lo; shi[t] = hi;
+    for (int k = 1; k <= 8 && base + k < L.levels; ++k) {
+        __syncthreads();
+        const uint32_t m = 256u >> k;
+        if (t < m) { lo = slo[2u * t]; hi = shi[2u * t]; box_union(lo, hi, slo[2u * t + 1u], shi[2u * t + 1u]); }
+        __syncthreads();
+        if (t < m) {
+            slo[t] = lo; shi[t] = hi;
+            const uint32_t e = blockIdx.x * m + t;
+            if (e < L.size[base + k]) { rlo[L.at[base + k] + e] = lo; rhi[L.at[base + k] + e] = hi; }
+        }
+    }
+}
+
+// Box and type mask of every binary node from the range tree. Most nodes cover two to four primitives:
+// a few adjacent loads. Bound by those loads; one thread per leaf climbing the tree, the second child to
+// arrive fitting the node, waited on a device-wide fence and an atomic at every node: 1.93 ms for
+// 300,000 triangles against 0.018 ms for the range tree and 0.015 ms for this.
+__global__ __launch_bounds__(256) void k_bvh_fit(RangeLevels L, uint32_t nodes, const uint32_t* __restrict__ first,
+                                                 const uint32_t* __restrict__ count, const float4* __restrict__ rlo,
+                                                 const float4* __restrict__ rhi, float4* __restrict__ nlo, float4* __restrict__ nhi,
+                                                 uint32_t* __restrict__ tmask) {
+    for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < nodes; i += gridDim.x * 256u) {
+        int32_t l = (int32_t)first[i], r = l + (int32_t)count[i] - 1;
+        const float inf = __builtin_inff();
+        float4 lo = make_float4(inf, inf, inf, 0.0f), hi = make_float4(-inf, -inf, -inf, 0.0f);
+        for (int k = 0; l <= r; ++k) {
+            if (l & 1) { box_union(lo, hi, rlo[L.at[k] + l], rhi[L.at[k] + l]); ++l; }
+            if (!(r & 1)) { box_union(lo, hi, rlo[L.at[k] + r], rhi[L.at[k] + r]); --r; }
+            l >>= 1; r >>= 1;
+        }
+        tmask[i] = __float_as_uint(lo.w);
+        nlo[i] = make_float4(lo.x, lo.y, lo.z, 0.0f);
+        nhi[i] = hi;
     }
 }
 
@@ -293,7 +323,7 @@ __device__ __forceinline__ uint32_t wave_exclusive(uint32_t v, uint32_t& total) 
 // 6. one level of the top-down collapse: output nodes [lb, le) (binary node of each in slot_b)
 // take their children; new interior children get the slots behind *counter (the next level)
 template <int WIDTH>
-__global__ __launch_bounds__(256) void k_bvh_collapse(Tree T, const uint32_t* __restrict__ level_base, int level,
+__global__ __launch_bounds__(256) void k_bvh_collapse(Tree T, uint32_t* __restrict__ level_base, int level,
                                                       int32_t* __restrict__ slot_b, uint32_t* __restrict__ counter,
                                                       float4* __restrict__ out, double* __restrict__ sah, float inv_root_area,
                                                       uint32_t* __restrict__ too_large) {
@@ -383,11 +413,13 @@ __global__ __launch_bounds__(256) void k_bvh_collapse(Tree T, const uint32_t* __
         if ((threadIdx.x & 63) == 0 && cost != 0.0) atomicAdd(sah, cost);
         if ((threadIdx.x & 63) == 0 && nleaf) atomicAdd(too_large + 1, nleaf);
     }
-}
-
-// end of a level: the next level's slots end where the counter stands
-__global__ void k_bvh_mark(const uint32_t* __restrict__ counter, uint32_t* __restrict__ level_base, int level) {
-    if (threadIdx.x == 0) level_base[level + 2] = *counter;
+    // end of a level: the next level's slots end where the counter stands once the level's last
+    // workgroup is done (a launch of its own for this cost 4 us a level and its gap)
+    __syncthreads();
+    if (threadIdx.x == 0 && atomicAdd(too_large + 2, 1u) == gridDim.x - 1u) {
+        level_base[level + 2] = atomicAdd(counter, 0u);
+        too_large[2] = 0u;
+    }
 }
 
 // 7. records in leaf order at each primitive's rank; leaf -> source index per type for the host
@@ -465,9 +497,12 @@ int gpu_build_scene(Context& C, const crt_scene_desc* d, uint32_t leaf, uint32_t
     Context* ctx = &C;
     // source records on the device
     DevBuf squads, sqbox, ssph, stris, snrm, suv, smap;
+    // work buffers come from and return to the context's cache (an allocation and its free cost 0.1-0.4 ms
+    // each, and a build takes thirty); large ones at their own size (the cache's classes are powers of two)
+    auto work = [&](DevBuf& b, size_t bytes) { return bytes <= (256ull << 20) ? b.alloc_cached(bytes, ctx) : b.alloc(bytes, ctx); };
     auto up = [&](DevBuf& b, const void* h, size_t bytes) -> int {
         if (!bytes) return CRT_OK;
-        int r = b.alloc(bytes, ctx);
+        int r = work(b, bytes);
         if (r) return r;
         HIP_TRY(ctx->stage.push(b.p, h, bytes, s));
         return CRT_OK;
@@ -482,21 +517,33 @@ int gpu_build_scene(Context& C, const crt_scene_desc* d, uint32_t leaf, uint32_t
     Prims P{dptr<float4>(squads), dptr<float4>(sqbox), dptr<float4>(ssph), dptr<float4>(stris), nq, ns, nt};
 
     // work buffers
-    DevBuf plo, phi, keys[2], vals[2], cb, cl, cr, parent, lparent, nlo, nhi, first, count, tmask, visits, tflags, ranks,
-        slot_b, level_base, counters, sah, nodes_tmp, tmp;
+    DevBuf plo, phi, keys[2], vals[2], cb, cl, cr, nlo, nhi, first, count, tmask, tflags, ranks, slot_b, level_base,
+        counters, sah, nodes_tmp, tmp, srcmap;
+    struct Drain {   // no buffer goes back while work on it is still queued, on error returns as well
+        hipStream_t s;
+        ~Drain() { (void)hipStreamSynchronize(s); }
+    } drain{s};
+    RangeLevels RL{};
+    uint64_t rn = 0;
+    for (uint64_t m = n; RL.levels < RangeLevels::kMax; m = (m + 1) / 2) {
+        RL.at[RL.levels] = (uint32_t)rn;
+        RL.size[RL.levels++] = (uint32_t)m;
+        rn += m;
+        if (m == 1) break;
+    }
     const size_t ni = std::max<uint32_t>(n - 1, 1);
-    if ((rc = plo.alloc((size_t)n * 16, ctx)) || (rc = phi.alloc((size_t)n * 16, ctx)) ||
-        (rc = keys[0].alloc((size_t)n * 8, ctx)) || (rc = keys[1].alloc((size_t)n * 8, ctx)) ||
-        (rc = vals[0].alloc((size_t)n * 4, ctx)) || (rc = vals[1].alloc((size_t)n * 4, ctx)) || (rc = cb.alloc(6 * 4, ctx)) ||
-        (rc = cl.alloc(ni * 4, ctx)) || (rc = cr.alloc(ni * 4, ctx)) || (rc = parent.alloc(ni * 4, ctx)) ||
-        (rc = lparent.alloc((size_t)n * 4, ctx)) || (rc = nlo.alloc(ni * 16, ctx)) || (rc = nhi.alloc(ni * 16, ctx)) ||
-        (rc = first.alloc(ni * 4, ctx)) || (rc = count.alloc(ni * 4, ctx)) || (rc = tmask.alloc(ni * 4, ctx)) ||
-        (rc = visits.alloc(ni * 4, ctx)) || (rc = tflags.alloc((size_t)n * sizeof(TypeCount), ctx)) ||
-        (rc = ranks.alloc((size_t)n * sizeof(TypeCount), ctx)) || (rc = slot_b.alloc(ni * 4, ctx)) ||
-        (rc = level_base.alloc((kMaxLevels + 2) * 4, ctx)) || (rc = counters.alloc(4 * 4, ctx)) || (rc = sah.alloc(8, ctx)))
+    if ((rc = work(plo, (size_t)n * 16)) || (rc = work(phi, (size_t)n * 16)) || (rc = work(keys[0], (size_t)n * 8)) ||
+        (rc = work(keys[1], (size_t)n * 8)) || (rc = work(vals[0], (size_t)n * 4)) || (rc = work(vals[1], (size_t)n * 4)) ||
+        (rc = work(cb, 6 * 4)) || (rc = work(cl, ni * 4)) || (rc = work(cr, ni * 4)) || (rc = work(nlo, ni * 16)) ||
+        (rc = work(nhi, ni * 16)) || (rc = work(first, ni * 4)) || (rc = work(count, ni * 4)) || (rc = work(tmask, ni * 4)) ||
+        (rc = work(tflags, (size_t)n * sizeof(TypeCount))) || (rc = work(ranks, (size_t)n * sizeof(TypeCount))) ||
+        (rc = work(slot_b, ni * 4)) ||
+        (rc = work(level_base, (kMaxLevels + 2) * 4)) || (rc = work(counters, 4 * 4)) || (rc = work(sah, 8)))
         return rc;
     const uint32_t per = width == 4 ? 8u : 4u;   // float4 per node
-    if ((rc = nodes_tmp.alloc(ni * per * 16, ctx))) return rc;
+    // the range tree is done with before the first output node is written: they share their memory
+    if ((rc = work(nodes_tmp, std::max<size_t>(ni * per * 16, rn * 32)))) return rc;
+    float4 *rlo = dptr<float4>(nodes_tmp), *rhi = rlo + rn;
     // temporary storage of the sort and the scan
     size_t sort_bytes = 0, scan_bytes = 0;
     HIP_TRY(hipcub::DeviceRadixSort::SortPairs(nullptr, sort_bytes, dptr<uint64_t>(keys[0]), dptr<uint64_t>(keys[1]),
@@ -504,12 +551,14 @@ int gpu_build_scene(Context& C, const crt_scene_desc* d, uint32_t leaf, uint32_t
     TypeCount zero{{0u, 0u, 0u}};
     HIP_TRY(hipcub::DeviceScan::ExclusiveScan(nullptr, scan_bytes, dptr<TypeCount>(tflags), dptr<TypeCount>(ranks),
                                               TypeCountAdd(), zero, (int)n, s));
-    if ((rc = tmp.alloc(std::max<size_t>(std::max(sort_bytes, scan_bytes), 16), ctx))) return rc;
+    if ((rc = work(tmp, std::max<size_t>(std::max(sort_bytes, scan_bytes), 16)))) return rc;
 
     // 1-2. boxes, centroid bounds, Morton codes, sort
     GB_LAUNCH(hipLaunchKernelGGL(k_fill_u32_gb, dim3(1), dim3(64), 0, s, dptr<uint32_t>(cb), 3u, 0xffffffffu), "fill");
     GB_LAUNCH(hipLaunchKernelGGL(k_fill_u32_gb, dim3(1), dim3(64), 0, s, dptr<uint32_t>(cb) + 3, 3u, 0u), "fill");
-    GB_LAUNCH(hipLaunchKernelGGL(k_bvh_bounds, dim3(grid_for(n, 2048)), dim3(256), 0, s, P, n, dptr<float4>(plo),
+    // two workgroups per CU: each ends in six atomics on the same words, 14 ns each one behind the other
+    // (300,000 triangles in 1,172 workgroups: 84 us)
+    GB_LAUNCH(hipLaunchKernelGGL(k_bvh_bounds, dim3(grid_for(n, 512)), dim3(256), 0, s, P, n, dptr<float4>(plo),
                                  dptr<float4>(phi), dptr<uint32_t>(cb)), "bounds");
     GB_LAUNCH(hipLaunchKernelGGL(k_bvh_morton, dim3(grid_for(n)), dim3(256), 0, s, dptr<float4>(plo), dptr<float4>(phi),
                                  dptr<uint32_t>(cb), n, dptr<uint64_t>(keys[0]), dptr<uint32_t>(vals[0])), "morton");
@@ -519,14 +568,13 @@ int gpu_build_scene(Context& C, const crt_scene_desc* d, uint32_t leaf, uint32_t
     const uint32_t* svals = dptr<uint32_t>(vals[1]);
     // 3-5. tree, boxes, ranks
     GB_LAUNCH(hipLaunchKernelGGL(k_bvh_karras, dim3(grid_for(n)), dim3(256), 0, s, skeys, (int)n, dptr<int32_t>(cl),
-                                 dptr<int32_t>(cr), dptr<int32_t>(parent), dptr<int32_t>(lparent), dptr<uint32_t>(first),
-                                 dptr<uint32_t>(count)), "karras");
-    GB_LAUNCH(hipLaunchKernelGGL(k_fill_u32_gb, dim3(grid_for(ni)), dim3(256), 0, s, dptr<uint32_t>(visits), (uint32_t)ni, 0u),
-              "fill");
-    GB_LAUNCH(hipLaunchKernelGGL(k_bvh_refit, dim3(grid_for(n)), dim3(256), 0, s, (int)n, svals, dptr<float4>(plo),
-                                 dptr<float4>(phi), dptr<int32_t>(cl), dptr<int32_t>(cr), dptr<int32_t>(parent),
-                                 dptr<int32_t>(lparent), dptr<float4>(nlo), dptr<float4>(nhi), dptr<uint32_t>(tmask),
-                                 dptr<uint32_t>(visits)), "refit");
+                                 dptr<int32_t>(cr), dptr<uint32_t>(first), dptr<uint32_t>(count)), "karras");
+    for (int base = 0; base < RL.levels; base += 8)
+        GB_LAUNCH(hipLaunchKernelGGL(k_bvh_range, dim3((RL.size[base] + 255u) / 256u), dim3(256), 0, s, RL, base, svals,
+                                     dptr<float4>(plo), dptr<float4>(phi), rlo, rhi), "range tree");
+    GB_LAUNCH(hipLaunchKernelGGL(k_bvh_fit, dim3(grid_for(ni)), dim3(256), 0, s, RL, (uint32_t)ni, dptr<uint32_t>(first),
+                                 dptr<uint32_t>(count), rlo, rhi, dptr<float4>(nlo), dptr<float4>(nhi),
+                                 dptr<uint32_t>(tmask)), "fit");
     GB_LAUNCH(hipLaunchKernelGGL(k_bvh_typeflags, dim3(grid_for(n)), dim3(256), 0, s, svals, P, n, dptr<TypeCount>(tflags)),
               "type flags");
     HIP_TRY(hipcub::DeviceScan::ExclusiveScan(tmp.p, scan_bytes, dptr<TypeCount>(tflags), dptr<TypeCount>(ranks),
@@ -537,7 +585,7 @@ int gpu_build_scene(Context& C, const crt_scene_desc* d, uint32_t leaf, uint32_t
     HIP_TRY(hipMemcpyAsync(&root_hi, dptr<float4>(nhi), 16, hipMemcpyDeviceToHost, s));
     const uint32_t init_base[3] = {0u, 1u, 1u};
     HIP_TRY(hipMemcpyAsync(dptr<uint32_t>(level_base), init_base, sizeof(init_base), hipMemcpyHostToDevice, s));
-    const uint32_t init_cnt[4] = {1u, 0u, 0u, 0u};   // node counter, too-large flag, leaves
+    const uint32_t init_cnt[4] = {1u, 0u, 0u, 0u};   // node counter, too-large flag, leaves, workgroups done
     HIP_TRY(hipMemcpyAsync(dptr<uint32_t>(counters), init_cnt, sizeof(init_cnt), hipMemcpyHostToDevice, s));
     const int32_t root_b = 0;
     HIP_TRY(hipMemcpyAsync(dptr<int32_t>(slot_b), &root_b, 4, hipMemcpyHostToDevice, s));
@@ -554,16 +602,16 @@ int gpu_build_scene(Context& C, const crt_scene_desc* d, uint32_t leaf, uint32_t
     int levels = 0;
     const uint32_t cgrid = grid_for(n / 2 + 1, 2048);
     for (int L = 0; L < kMaxLevels; ++L) {
+        // at most width^L nodes in level L
+        const uint32_t lgrid = L < 10 ? std::min(cgrid, grid_for(1ull << (width == 4 ? 2 * L : L))) : cgrid;
         if (width == 4)
-            GB_LAUNCH(hipLaunchKernelGGL(k_bvh_collapse<4>, dim3(cgrid), dim3(256), 0, s, T, dptr<uint32_t>(level_base), L,
+            GB_LAUNCH(hipLaunchKernelGGL(k_bvh_collapse<4>, dim3(lgrid), dim3(256), 0, s, T, dptr<uint32_t>(level_base), L,
                                          dptr<int32_t>(slot_b), dptr<uint32_t>(counters), dptr<float4>(nodes_tmp),
                                          dptr<double>(sah), 1.0f / root_area, dptr<uint32_t>(counters) + 1), "collapse");
         else
-            GB_LAUNCH(hipLaunchKernelGGL(k_bvh_collapse<2>, dim3(cgrid), dim3(256), 0, s, T, dptr<uint32_t>(level_base), L,
+            GB_LAUNCH(hipLaunchKernelGGL(k_bvh_collapse<2>, dim3(lgrid), dim3(256), 0, s, T, dptr<uint32_t>(level_base), L,
                                          dptr<int32_t>(slot_b), dptr<uint32_t>(counters), dptr<float4>(nodes_tmp),
                                          dptr<double>(sah), 1.0f / root_area, dptr<uint32_t>(counters) + 1), "collapse");
-        GB_LAUNCH(hipLaunchKernelGGL(k_bvh_mark, dim3(1), dim3(64), 0, s, dptr<uint32_t>(counters), dptr<uint32_t>(level_base), L),
-                  "mark");
         if ((L & 7) == 7 || L == kMaxLevels - 1) {
             HIP_TRY(hipMemcpyAsync(lb.data(), level_base.p, lb.size() * 4, hipMemcpyDeviceToHost, s));
             HIP_TRY(hipStreamSynchronize(s));
@@ -598,8 +646,7 @@ int gpu_build_scene(Context& C, const crt_scene_desc* d, uint32_t leaf, uint32_t
     if (nt && !src.tri_normals.empty() && (rc = sc.tri_normals.alloc((size_t)nt * 48, ctx))) return rc;
     if (nt && !src.tri_uvs.empty() && (rc = sc.tri_uvs.alloc((size_t)nt * 24, ctx))) return rc;
     if (ns && (rc = sc.sphere_map.alloc((size_t)ns * 24, ctx))) return rc;
-    DevBuf srcmap;
-    if ((rc = srcmap.alloc((size_t)(nt + ns + nq) * 4 + 16, ctx))) return rc;
+    if ((rc = work(srcmap, (size_t)(nt + ns + nq) * 4 + 16))) return rc;
     uint32_t* src_tri = dptr<uint32_t>(srcmap);
     uint32_t* src_sph = src_tri + nt;
     uint32_t* src_quad = src_sph + ns;
