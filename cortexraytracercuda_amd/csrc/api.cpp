@@ -569,7 +569,7 @@ uint64_t Job::bytes_needed(const crt_render_desc& r) {
     return npix * 16 + npix * 3 + 16 + (r.rng_mode == CRT_RNG_MINSTD ? npix * 4 : 0);
 }
 
-int Job::setup(Context* ctx, DeviceScene* sc, const crt_render_desc& r, hipStream_t st) {
+int Job::setup(Context* ctx, DeviceScene* sc, const crt_render_desc& r, hipStream_t st, bool later) {
     rd = r;
     scene = sc;
     npix = r.width * r.height;
@@ -589,8 +589,12 @@ int Job::setup(Context* ctx, DeviceScene* sc, const crt_render_desc& r, hipStrea
     if (r.rng_mode == CRT_RNG_MINSTD && (rc = rng.alloc_cached((size_t)npix * 4, ctx))) return rc;
     req.accum = (float*)accum.p;
     req.rng_state = (uint32_t*)rng.p;
-    if (crt_k_init_request(st ? st : ctx->stream, (float4*)accum.p, (uint32_t*)rng.p, r.width, r.height, r.seed) ||
-        crt_k_fill_u32(st ? st : ctx->stream, (uint32_t*)rays_counter(), 2, 0u))
+    return later ? CRT_OK : init(st ? st : ctx->stream);
+}
+
+int Job::init(hipStream_t st) {
+    if (crt_k_init_request(st, (float4*)accum.p, (uint32_t*)rng.p, rd.width, rd.height, rd.seed) ||
+        crt_k_fill_u32(st, (uint32_t*)rays_counter(), 2, 0u))
         return set_error(CRT_ERR_HIP, "init kernel launch failed");
     return CRT_OK;
 }
@@ -646,6 +650,11 @@ bool Job::take_whole(uint32_t cap, WorkItem& w) {
 
 uint32_t WorkItem::whole_ids() const {
     return job->rd.rng_mode == CRT_RNG_MINSTD ? pix_count : pix_count * sample_count;
+}
+
+bool WorkItem::same_kernel(const WorkItem& w) const {
+    const HostScene &a = job->scene->host, &b = w.job->scene->host;
+    return job->rd.rng_mode == w.job->rd.rng_mode && !a.num_instances == !b.num_instances && !a.num_shapes == !b.num_shapes;
 }
 
 // Runs one fused pass over the given work items (all with the same rng mode). Asynchronous on
@@ -787,7 +796,7 @@ int Context::run_whole(std::vector<WorkItem>& items, const PassBufs& B) {
     pass_parity ^= 1;
     HIP_TRY(hipEventSynchronize(req_event[buf]));
     crt_dev_request* host = (crt_dev_request*)req_host[buf];
-    uint32_t base = 0;
+    uint32_t base = 0, end = 0;
     for (size_t k = 0; k < items.size(); ++k) {
         const WorkItem& w = items[k];
         crt_dev_request r = w.job->req;
@@ -795,10 +804,11 @@ int Context::run_whole(std::vector<WorkItem>& items, const PassBufs& B) {
         r.pix_begin = w.pix_begin; r.pix_count = w.pix_count;
         r.sample_begin = w.sample_begin; r.sample_count = w.sample_count;
         host[k] = r;
-        base += w.whole_ids();
+        end = base + w.whole_ids();
+        base = whole_span(end);
         w.job->rays_in_flight += (uint64_t)w.pix_count * w.sample_count;
     }
-    if (base > B.pass_ids) return set_error(CRT_ERR_INTERNAL, "pass exceeds the pass capacity");
+    if (end > B.pass_ids) return set_error(CRT_ERR_INTERNAL, "pass exceeds the pass capacity");
     crt_dev_request* dreq = B.req[buf];
     HIP_TRY(hipMemcpyAsync(dreq, host, sizeof(crt_dev_request) * items.size(), hipMemcpyHostToDevice, stream));
     if (crt_k_fill_u32(stream, B.next, (uint32_t)items.size(), 0u)) return set_error(CRT_ERR_HIP, "fill launch failed");
@@ -809,16 +819,23 @@ int Context::run_whole(std::vector<WorkItem>& items, const PassBufs& B) {
     const uint64_t wave_words = 64ull * crt_k_paths_overflow_entries();
     const uint64_t waves = B.gstack_words / K / wave_words;
     if (waves == 0) return set_error(CRT_ERR_INTERNAL, "traversal stacks too small");
-    for (size_t k = 0; k < items.size(); ++k) {
+    uint32_t q = 0;
+    for (size_t k = 0, m; k < items.size(); k = m, q = (q + 1) % K) {
         const WorkItem& w = items[k];
-        const uint32_t q = (uint32_t)(k % K);
+        uint32_t span = w.whole_ids(), max_pix = w.pix_count;
+        for (m = k + 1; m < items.size() && items[m].same_kernel(w); ++m) {
+            const uint32_t s2 = host[m].path_base - host[k].path_base + items[m].whole_ids();
+            if (s2 > CRT_PATHS_MERGE || s2 > waves * CRT_PATHS_ALIGN) break;
+            span = s2;
+            max_pix = std::max(max_pix, items[m].pix_count);
+        }
         hipStream_t s = q == 0 ? stream : sub_stream[q - 1];
         const HostScene& H = w.job->scene->host;
         if (crt_k_paths(s, (int)w.job->rd.rng_mode, H.num_instances ? 1 : 0, H.num_shapes ? 1 : 0,
                         (uint32_t)std::min<uint64_t>(waves, 1u << 20), (const crt_dev_scene*)scene_table.p, dreq + k,
-                        w.whole_ids(), B.next + k, B.out_rad + host[k].path_base, B.gstack + q * waves * wave_words, B.counters))
+                        (uint32_t)(m - k), span, B.next + k, B.out_rad + host[k].path_base, B.gstack + q * waves * wave_words, B.counters))
             return set_error(CRT_ERR_HIP, "path launch failed");
-        if (w.job->rd.rng_mode == CRT_RNG_PCG && crt_k_resolve(s, dreq + k, 1, w.pix_count, B.out_rad, nullptr))
+        if (w.job->rd.rng_mode == CRT_RNG_PCG && crt_k_resolve(s, dreq + k, (int)(m - k), max_pix, B.out_rad, nullptr))
             return set_error(CRT_ERR_HIP, "resolve launch failed");
     }
     for (uint32_t q = 1; q < K; ++q) {
@@ -915,7 +932,7 @@ int Context::render_jobs(std::vector<Job*>& jobs, bool time_stages, crt_stats* s
             WorkItem w;
             if (cap == 0 || items.size() >= B.max_requests) break;
             if (!whole(j) || !j->take_whole(cap, w)) continue;
-            cap -= w.whole_ids();
+            cap -= std::min(cap, whole_span(w.whole_ids()));
             paths += (uint64_t)w.pix_count * w.sample_count;
             items.push_back(w);
         }

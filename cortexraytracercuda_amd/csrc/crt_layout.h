@@ -114,6 +114,9 @@ struct crt_dev_request {
     uint32_t sample_begin, sample_count;
     float* accum;            // float4 per pixel (rgb sums, sample count), rows top-down
     uint32_t* rng_state;     // MINSTD: per-pixel engine state carried across samples
+    // whole-path launches add the request's closest-hit queries here (may be null); the top bit marks
+    // a traversal stack overflow
+    unsigned long long* rays;
     uint32_t ortho;          // 1: orthographic camera
     uint32_t pad;
 };

@@ -100,7 +100,12 @@ struct WorkItem {
     uint32_t pix_begin = 0, pix_count = 0, sample_begin = 0, sample_count = 0;
     // path ids of a whole-path launch (a MINSTD pixel's samples run one after the other in one id)
     uint32_t whole_ids() const;
+    // one whole-path launch can take both
+    bool same_kernel(const WorkItem& w) const;
 };
+
+// Path ids a work item takes up in the id space of whole-path launches.
+inline uint32_t whole_span(uint32_t ids) { return (ids + CRT_PATHS_ALIGN - 1u) & ~(CRT_PATHS_ALIGN - 1u); }
 
 struct Job {
     crt_render_desc rd{};
@@ -115,7 +120,9 @@ struct Job {
     }
     static int validate(const crt_render_desc& r);
     static uint64_t bytes_needed(const crt_render_desc& r);
-    int setup(Context* ctx, DeviceScene* sc, const crt_render_desc& r, hipStream_t st = nullptr);
+    // buffers, and init() on `st` (the context's stream) unless `later`
+    int setup(Context* ctx, DeviceScene* sc, const crt_render_desc& r, hipStream_t st = nullptr, bool later = false);
+    int init(hipStream_t st);
     // a job whose accumulation buffer the caller owns (device memory): no allocation
     void setup_external(DeviceScene* sc, const crt_render_desc& r, float* accum_dev);
     bool take(uint32_t cap, WorkItem& w);
@@ -144,6 +151,10 @@ struct ServeReq {
     int lane = 0;                  // open pass (server lane) that traces all of its segments
     uint64_t load = 0;             // paths it adds to its lane's load until it completes
     hipEvent_t ev_done = nullptr;
+    // whole-path launches: the lanes that have its buffers' start behind them, and the number (from 1)
+    // of its last launch on each
+    uint32_t lanes_seen = 0;
+    uint64_t last[2] = {0, 0};
 };
 
 // One segment (work item) of a request inside the server's open pass: a request-table entry.
@@ -191,6 +202,10 @@ struct Server {
     static constexpr int kVariants = 8;
     uint32_t warm[kVariants] = {};                 // eager iterations per variant (graphs are captured after kRing)
     hipGraphExec_t graph[kVariants][kRing] = {};   // [variant][snapshot slot]
+    // whole-path launches: enqueued / finished (events in ev), path ids of those in flight
+    static constexpr uint32_t kLaunchEntries = kEntries / kRing;   // requests of one launch at most
+    uint64_t launched = 0, landed = 0, ids_ahead = 0;
+    uint32_t launch_ids[kRing] = {};
 };
 
 struct Context {
@@ -269,6 +284,8 @@ struct Context {
     // up to kSrvLanes open passes on their own streams (each with a share of the slot pool), so one
     // pass's drain tail overlaps the other's full launches; a request's segments stay in one lane
     static constexpr int kSrvLanes = 2;
+    // path ids of one whole-path launch of the serving loop
+    static constexpr uint32_t kServeLaunch = 1u << 22, kServeStreams = 1u << 18;
     Server srv[kSrvLanes];
     uint32_t srv_lanes = 1;
     uint64_t lane_load[kSrvLanes] = {};
@@ -306,7 +323,7 @@ struct Context {
     int submit(crt_scene_id scene, const crt_render_desc* rd, crt_request_id* out);
     void server_loop();
     void server_copy_loop();
-    void server_complete(ServeReq* r, int status);
+    void server_complete(const std::vector<std::pair<ServeReq*, int>>& done);
     void stop_server();
     int server_init();
     int server_init_lane(Server& S, uint32_t slots, uint32_t cap, bool first);
@@ -315,6 +332,14 @@ struct Context {
     void server_release_lane(Server& S);
     int server_iteration(Server& S);
     int server_append(Server& S, std::vector<ServeReq*>& act);
+    // served requests run as whole-path launches, as blocking renders do (else as iterations of open passes)
+    bool serve_whole() const { return !staged && bvh_width == 4u; }
+    std::vector<ServeReq*> serving_order(const std::vector<ServeReq*>& act, uint32_t& rr) const;
+    int launch_whole(const std::vector<ServeReq*>& act, bool& any_step);
+    int launch_group(uint32_t lane, std::vector<std::pair<ServeReq*, WorkItem>>& group);
+    int finish_whole(uint32_t lane, ServeReq* r);
+    int after_others(uint32_t lane, const ServeReq* r);
+    int land_launches(bool wait, bool& any_step);
     bool append_segment(Server& S, ServeReq* r, uint32_t seg_cap);
     int server_process_snapshot(Server& S, std::vector<ServeReq*>& act);
     void server_reset_pass(Server& S);

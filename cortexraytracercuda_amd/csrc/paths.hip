@@ -30,8 +30,8 @@ __device__ __forceinline__ uint32_t lane_rank(uint64_t mask) {
     return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
 }
 
-// Follows the paths of one request (ids [0, total): its pixels, each pixel's samples consecutive) to
-// their end in one launch. A workgroup is one wave. Each round the wave holds at most `group` paths,
+// Follows the paths of one request (ids [0, total): its pixels, each pixel's samples consecutive), or of
+// several short ones, to their end in one launch. A workgroup is one wave. Each round the wave holds at most `group` paths,
 // one per lane, and traces and shades one segment of each:
 //   - lanes whose path ended take a path from the wave's queue in LDS;
 //   - when queue and live paths together no longer fill a group, the live ones are put in the queue
@@ -48,10 +48,11 @@ __device__ __forceinline__ uint32_t lane_rank(uint64_t mask) {
 // MINSTD: an id is a pixel; its samples run one after the other in its lane, each ended path starting
 // the next sample, and are added to the accumulation buffer in order (a scene file's 512x388, 49
 // samples, depth 100: 61 -> 5.7 ms against one staged pass per sample).
-template <int MODE, int TL>
+template <int MODE, int TL, bool MERGED>
 __global__ __launch_bounds__(64, kWaves) void k_paths(const crt_dev_scene* __restrict__ scenes,
-                                                           const crt_dev_request* __restrict__ req, uint32_t total,
-                                                           uint32_t group, uint32_t chunk, uint32_t* __restrict__ next,
+                                                           const crt_dev_request* __restrict__ reqs, uint32_t nreq,
+                                                           uint32_t total, uint32_t group, uint32_t chunk,
+                                                           uint32_t* __restrict__ next,
                                                            float4* __restrict__ out_rad, uint32_t* __restrict__ gstack,
                                                            crt_dev_counters* __restrict__ counters) {
     constexpr bool STREAM = MODE == CRT_RNG_MINSTD;
@@ -60,13 +61,33 @@ __global__ __launch_bounds__(64, kWaves) void k_paths(const crt_dev_scene* __res
     __shared__ uint32_t s_wait[(STREAM ? 13 : 12) * 64];
     __shared__ uint32_t s_path[6 * 64];
     const uint32_t lane = threadIdx.x;
-    const crt_dev_request& R = *req;
+    bool more = true;
+    uint32_t cur = min(blockIdx.x * chunk, total);
+    if (MERGED) {
+        // one group of ids a wave, none handed out
+        more = false;
+        cur = blockIdx.x * group;
+        const uint32_t base = reqs->path_base;
+        uint32_t lo = 0, hi = nreq;
+        while (hi - lo > 1) {
+            const uint32_t mid = (lo + hi) >> 1;
+            if (reqs[mid].path_base - base <= cur) lo = mid; else hi = mid;
+        }
+        reqs += lo;
+        cur -= reqs->path_base - base;
+        out_rad += reqs->path_base - base;
+        total = STREAM ? reqs->pix_count : reqs->pix_count * reqs->sample_count;
+        cur = min(cur, total);
+    }
+    uint32_t end = min(cur + chunk, total);
+    const crt_dev_request& R = *reqs;
     const crt_dev_scene* sc = scenes + R.scene;
     const SceneView S = scene_view(sc);
     const GSlot gst{gstack, (blockIdx.x * 64u + lane) * kOverflow};
-    uint64_t nrays = 0, nretrace = 0, novf = 0, nexact = 0, nlight = 0;   // wave totals (scalar)
-    uint32_t waiting = 0, cur = min(blockIdx.x * chunk, total), end = min(cur + chunk, total);
-    bool more = true, live = false;
+    uint64_t cn[5] = {0,0,0,0,0};
+    auto count = [&](int k, uint64_t mask) { cn[k] += (uint64_t)__popcll(mask); };
+    uint32_t waiting = 0;
+    bool live = false;
     V3 o = v3(0.0f, 0.0f, 0.0f), d = o, att = o;
     uint32_t pix = 0, sample = 0, state = 0, ms = 0;
     auto start = [&]() {
@@ -126,7 +147,7 @@ __global__ __launch_bounds__(64, kWaves) void k_paths(const crt_dev_scene* __res
         __syncthreads();
         const uint64_t am = __ballot(live);
         if (!am) break;
-        nrays += (uint64_t)__popcll(am);
+        count(0, am);
         uint32_t pf = 0, lt = 0, ovf = 0, exact = 0;
         if (live) {
             // what the traversal does not need waits in LDS: held in registers across it, the loop spills
@@ -179,17 +200,23 @@ __global__ __launch_bounds__(64, kWaves) void k_paths(const crt_dev_scene* __res
         }
         // counted where the wave has come together again: a ballot inside the branch sees the lanes
         // of one way through it only
-        novf += (uint64_t)__popcll(__ballot(ovf != 0u));
-        nexact += (uint64_t)__popcll(__ballot(exact != 0u));
-        nretrace += (uint64_t)__popcll(__ballot(pf != 0u));
-        nlight += (uint64_t)__popcll(__ballot(lt != 0u)) * sc->num_lights;
+        count(1, __ballot(pf != 0u));
+        count(2, __ballot(lt != 0u));
+        count(3, __ballot(ovf != 0u));
+        count(4, __ballot(exact != 0u));
     }
     if (lane == 0) {
-        atomicAdd(&counters->rays, (unsigned long long)nrays);
-        if (nretrace) atomicAdd(&counters->retraces, (unsigned long long)nretrace);
-        if (nlight) atomicAdd(&counters->light_tests, (unsigned long long)nlight);
-        if (novf) atomicAdd(&counters->stack_overflow, (unsigned long long)novf);
-        if (nexact) atomicAdd(&counters->exact, (unsigned long long)nexact);
+        const unsigned long long nrays = cn[0], nretrace = cn[1], nlight = cn[2] * sc->num_lights, novf = cn[3],
+                                 nexact = cn[4];
+        atomicAdd(&counters->rays, nrays);
+        if (nretrace) atomicAdd(&counters->retraces, nretrace);
+        if (nlight) atomicAdd(&counters->light_tests, nlight);
+        if (novf) atomicAdd(&counters->stack_overflow, novf);
+        if (nexact) atomicAdd(&counters->exact, nexact);
+        if (R.rays) {
+            atomicAdd(R.rays, nrays + nretrace);
+            if (novf) atomicOr(R.rays, 1ull << 63);
+        }
     }
 }
 
@@ -208,18 +235,19 @@ template <typename K> uint32_t resident_waves(K kernel) {
 extern "C" uint32_t crt_k_paths_overflow_entries(void) { return (uint32_t)kOverflow; }
 
 extern "C" int crt_k_paths(hipStream_t s, int rng_mode, int two_level, int shapes, uint32_t max_waves, const crt_dev_scene* scenes,
-                           const crt_dev_request* req, uint32_t total, uint32_t* next, float4* out_rad, uint32_t* gstack,
-                           crt_dev_counters* counters) {
+                           const crt_dev_request* reqs, uint32_t nreq, uint32_t total, uint32_t* next, float4* out_rad,
+                           uint32_t* gstack, crt_dev_counters* counters) {
     if (total == 0) return 0;
+    if (nreq > 1 && (total > CRT_PATHS_MERGE || total > (uint64_t)max_waves * CRT_PATHS_ALIGN)) return (int)hipErrorInvalidValue;
     auto launch = [&](auto kfn, uint32_t resident) {
         uint32_t waves = resident < max_waves ? resident : max_waves;
         // A launch with fewer paths than lanes is cut into groups of 32, not 64: twice the waves, each
         // done when the longest of half as many rays is (box 64^2 16 spp 0.175 -> 0.165 ms GPU). 16 and
         // 8 cost more waves' worth of instructions than they save (0.21 ms).
-        uint32_t group = 64u;
+        uint32_t group = CRT_PATHS_ALIGN;
         if (group > kMinGroup && (uint64_t)waves * kMinGroup >= total) group = kMinGroup;
         const uint32_t groups = (total + group - 1u) / group;
-        if (waves > groups) waves = groups;
+        if (waves > groups || nreq > 1) waves = groups;
         // Groups per hand-out: large enough that the counter's atomics (about 14 ns each, one after
         // the other across the XCDs) do not bound the launch, small enough that the waves in flight
         // trace neighbouring pixels (large frame at 1, 4, 8, 16, 32 groups: 29.6, 20.8, 21.5, 23.6,
@@ -227,12 +255,13 @@ extern "C" int crt_k_paths(hipStream_t s, int rng_mode, int two_level, int shape
         // the waves end together.
         uint32_t c = groups / (waves * 8u);
         c = c < 1u ? 1u : (c > kMaxChunk ? kMaxChunk : c);
-        hipLaunchKernelGGL(kfn, dim3(waves), dim3(64), 0, s, scenes, req, total, group, c * group, next, out_rad, gstack, counters);
+        hipLaunchKernelGGL(kfn, dim3(waves), dim3(64), 0, s, scenes, reqs, nreq, total, group, nreq > 1 ? group : c * group, next, out_rad, gstack, counters);
     };
 #define CRT_PTH(M, T)                                                         \
     {                                                                         \
-        static const uint32_t resident = resident_waves(k_paths<M, T>);       \
-        launch(k_paths<M, T>, resident);                                      \
+        static const uint32_t resident = resident_waves(k_paths<M, T, false>); \
+        if (nreq > 1) launch(k_paths<M, T, true>, resident);                  \
+        else launch(k_paths<M, T, false>, resident);                          \
     }
 #define CRT_PTH_T(M)                                                          \
     {                                                                         \

@@ -6,15 +6,22 @@
 //   - requests are admitted first-fit against the HBM budget (accumulation, tonemap and RNG
 //     buffers; scenes are already resident and counted at upload) and join the lane with the
 //     fewest outstanding paths;
-//   - an admitted request is cut into segments (pixel range x sample range); a segment becomes a
-//     request-table entry of its lane's open pass and its path ids are appended behind the pass's
-//     last id between two iterations, so the next regeneration stage already starts its camera
-//     rays among the paths of every other request in flight;
+//   - an admitted request is cut into segments (pixel range x sample range) of up to 4 M paths; a
+//     segment is one launch that follows its paths to their end, and its resolve, on the lane with
+//     the fewest paths ahead; the next ones are enqueued while fewer than two launches' worth are.
+//     Segments of one request are resolved in sample order by events between the lanes; after the
+//     last one comes the tonemap, and a completion thread reads the image back;
+//   - short segments of several requests share a launch.
+// One request's paths no longer wait for the others' between bounces as in the iterations below, and
+// their state stays off HBM: SERVE_FIGURES.
+// Contexts whose renders run in stages (two-wide nodes, a closest-hit stage asked for) serve in stages:
+//   - a segment becomes a request-table entry of its lane's open pass and its path ids are appended
+//     behind the pass's last id between two iterations, so the next regeneration stage already starts
+//     its camera rays among the paths of every other request in flight;
 //   - path ids are generated in order and every live path is shaded once per iteration: once the
 //     generated count and the smallest surviving id (left by the shade stage) have passed a
 //     segment's last id, the host enqueues its resolve (segments of one request in order), and
-//     after the last one the tonemap; a completion thread reads the image back, so a request
-//     completes independently of the others;
+//     after the last one the tonemap;
 //   - when a pass has no room left (path ids or table entries) it drains and starts over.
 // Results do not depend on the mix: streams are keyed per (seed, pixel, sample, bounce) and each
 // pixel's samples are summed in sample order whatever the segment boundaries are.
@@ -192,7 +199,7 @@ bool Context::server_idle() {
     if (!srv_waiting.empty() || !srv_active.empty()) return false;
     for (uint32_t l = 0; l < (uint32_t)kSrvLanes; ++l) {
         const Server& S = srv[l];
-        if (S.ready && ((uint64_t)S.total > S.done_paths || S.processed < S.iter)) return false;
+        if (S.ready && ((uint64_t)S.total > S.done_paths || S.processed < S.iter || S.landed < S.launched)) return false;
     }
     return true;
 }
@@ -245,31 +252,35 @@ bool Context::append_segment(Server& S, ServeReq* r, uint32_t seg_cap) {
     return true;
 }
 
-// Appends segments of active requests to the open pass while the backlog of ungenerated path ids
-// is below two slot pools (a new request starts within a few iterations). MINSTD requests keep at
-// most one segment in flight (each pixel's engine advances sample after sample).
 // Order (CRT_SERVE_SMALL_THEN_OLDEST, the default): requests with at most serve_small path ids left,
-// in admission order, then the others oldest first, each appending segments while the backlog
-// allows. Draining the large requests in arrival order bounds the largest latency of a loop that
-// is offered more work than it renders (the last request to finish is then one that arrived late);
-// small requests pass them, finish within a few iterations and keep the median low.
+// in admission order, then the others oldest first. Draining the large requests in arrival order
+// bounds the largest latency of a loop that is offered more work than it renders (the last request to
+// finish is then one that arrived late); small requests pass them and keep the median low.
 // CRT_SERVE_ROUND_ROBIN: one segment per request and call in rotating order (every request
 // progresses; the large ones finish last whenever they arrived).
-int Context::server_append(Server& S, std::vector<ServeReq*>& act) {
-    if (act.empty() || S.full) return CRT_OK;
-    const uint32_t seg_cap = std::max<uint32_t>(S.slots / 2, 1u);
-    const uint32_t n0 = (uint32_t)S.entries.size();
-    const size_t na = act.size();
+std::vector<ServeReq*> Context::serving_order(const std::vector<ServeReq*>& act, uint32_t& rr) const {
     std::vector<ServeReq*> order;
+    const size_t na = act.size();
     order.reserve(na);
-    const bool rr = serve_order == CRT_SERVE_ROUND_ROBIN;
-    if (rr) {
-        for (size_t t = 0; t < na; ++t) order.push_back(act[(S.rr + t) % na]);
-        S.rr++;
+    if (serve_order == CRT_SERVE_ROUND_ROBIN) {
+        for (size_t t = 0; t < na; ++t) order.push_back(act[(rr + t) % na]);
+        rr++;
     } else {
         for (ServeReq* r : act) if (r->job->paths_left() <= serve_small) order.push_back(r);
         for (ServeReq* r : act) if (r->job->paths_left() > serve_small) order.push_back(r);
     }
+    return order;
+}
+
+// Appends segments of active requests to the open pass while the backlog of ungenerated path ids
+// is below two slot pools (a new request starts within a few iterations). MINSTD requests keep at
+// most one segment in flight (each pixel's engine advances sample after sample).
+int Context::server_append(Server& S, std::vector<ServeReq*>& act) {
+    if (act.empty() || S.full) return CRT_OK;
+    const uint32_t seg_cap = std::max<uint32_t>(S.slots / 2, 1u);
+    const uint32_t n0 = (uint32_t)S.entries.size();
+    const bool rr = serve_order == CRT_SERVE_ROUND_ROBIN;
+    const std::vector<ServeReq*> order = serving_order(act, S.rr);
     bool stop = false;
     for (ServeReq* r : order) {
         if (stop) break;
@@ -431,44 +442,222 @@ int Context::server_process_snapshot(Server& S, std::vector<ServeReq*>& act) {
     return CRT_OK;
 }
 
-// Readback and completion of one finished request (completion thread; status != CRT_OK: no copies).
-void Context::server_complete(ServeReq* r, int st) {
+// ------------------------------------------------------------------ whole-path launches
+// What the lane's stream does next on the request waits for its launches still in flight on the others.
+// (A launch's event may be recorded anew once the launch has landed: it is not waited for then.)
+int Context::after_others(uint32_t lane, const ServeReq* r) {
+    for (uint32_t l = 0; l < srv_lanes; ++l)
+        if (l != lane && r->last[l] > srv[l].landed)
+            HIP_TRY(hipStreamWaitEvent(srv[lane].s, srv[l].ev[(r->last[l] - 1) % Server::kRing], 0));
+    return CRT_OK;
+}
+
+// Enqueues the tonemap of a request whose segments are all on the device (none for a cancelled one)
+// behind them on every lane, and its completion event.
+int Context::finish_whole(uint32_t lane, ServeReq* r) {
+    Server& S = srv[lane];
+    int rc = after_others(lane, r);
+    if (rc) return rc;
+    if (!r->cancel) {
+        if (r->segs == 0 && (rc = r->job->init(S.s))) return rc;   // a request without samples
+        if (crt_k_tonemap(S.s, (const float4*)r->job->accum.p, r->job->npix, r->job->rd.spp, (uint8_t*)r->job->rgb.p))
+            return set_error(CRT_ERR_HIP, "tonemap launch failed");
+    }
+    if (!r->ev_done) HIP_TRY(hipEventCreateWithFlags(&r->ev_done, hipEventDisableTiming));
+    HIP_TRY(hipEventRecord(r->ev_done, S.s));
+    r->finishing = true;
+    return CRT_OK;
+}
+
+// One launch of the segments in `group` on the lane's stream, and their resolve. The radiance of every
+// launch lies at the start of the lane's buffer: the stream orders it behind the resolve before it.
+int Context::launch_group(uint32_t lane, std::vector<std::pair<ServeReq*, WorkItem>>& group) {
+    Server& S = srv[lane];
+    const int slot = (int)(S.launched % Server::kRing);
+    const size_t e0 = (size_t)slot * Server::kLaunchEntries;
+    crt_dev_request* dreq = (crt_dev_request*)S.req.p + e0;
+    uint32_t end = 0, max_pix = 0;
+    uint64_t ids = 0;
+    int rc;
+    for (size_t k = 0; k < group.size(); ++k) {
+        ServeReq* r = group[k].first;
+        const WorkItem& w = group[k].second;
+        crt_dev_request q = r->job->req;
+        q.path_base = whole_span(end);
+        q.pix_begin = w.pix_begin; q.pix_count = w.pix_count;
+        q.sample_begin = w.sample_begin; q.sample_count = w.sample_count;
+        q.rays = r->job->rays_counter();
+        S.req_host[e0 + k] = q;
+        end = q.path_base + w.whole_ids();
+        max_pix = std::max(max_pix, w.pix_count);
+        ids += (uint64_t)w.pix_count * w.sample_count;
+        // the first launch starts the request's buffers, the other lane's launches come behind that
+        if (r->segs == 0) {
+            if ((rc = r->job->init(S.s))) return rc;
+            if (!r->ev_done) HIP_TRY(hipEventCreateWithFlags(&r->ev_done, hipEventDisableTiming));
+            HIP_TRY(hipEventRecord(r->ev_done, S.s));
+        } else if (!(r->lanes_seen >> lane & 1u)) {
+            HIP_TRY(hipStreamWaitEvent(S.s, r->ev_done, 0));
+        }
+        r->lanes_seen |= 1u << lane;
+    }
+    if (end > S.cap) return set_error(CRT_ERR_INTERNAL, "launch exceeds the lane's path ids");
+    const WorkItem& w0 = group[0].second;
+    const HostScene& H = w0.job->scene->host;
+    const uint64_t waves = S.gstack.bytes / sizeof(uint32_t) / (64ull * crt_k_paths_overflow_entries());
+    uint32_t* next = (uint32_t*)S.live_min.p;
+    HIP_TRY(hipMemcpyAsync(dreq, S.req_host + e0, sizeof(crt_dev_request) * group.size(), hipMemcpyHostToDevice, S.s));
+    if (crt_k_fill_u32(S.s, next, 1u, 0u)) return set_error(CRT_ERR_HIP, "fill launch failed");
+    if (crt_k_paths(S.s, (int)w0.job->rd.rng_mode, H.num_instances ? 1 : 0, H.num_shapes ? 1 : 0,
+                    (uint32_t)std::min<uint64_t>(waves, 1u << 20), (const crt_dev_scene*)scene_table.p, dreq,
+                    (uint32_t)group.size(), end, next, (float4*)S.out_rad.p, (uint32_t*)S.gstack.p, (crt_dev_counters*)S.counters.p))
+        return set_error(CRT_ERR_HIP, "path launch failed");
+    if (w0.job->rd.rng_mode == CRT_RNG_PCG) {
+        // segments of one request are resolved in sample order, whichever lanes traced them
+        for (auto& g : group)
+            if ((rc = after_others(lane, g.first))) return rc;
+        if (crt_k_resolve(S.s, dreq, (int)group.size(), max_pix, (const float4*)S.out_rad.p, nullptr))
+            return set_error(CRT_ERR_HIP, "resolve launch failed");
+    }
+    for (auto& g : group) {
+        ServeReq* r = g.first;
+        r->last[lane] = S.launched + 1;
+        r->segs++;
+        r->timing.passes++;
+        if (r->timing.first_pass_s == 0.0) r->timing.first_pass_s = now_s();
+        if (r->job->scheduled_all() && (rc = finish_whole(lane, r))) return rc;
+    }
+    // behind the tonemaps: a landed launch's finished requests can be read back
+    HIP_TRY(hipEventRecord(S.ev[slot], S.s));
+    S.launch_ids[slot] = (uint32_t)std::min<uint64_t>(ids, 0xffffffffu);
+    S.ids_ahead += S.launch_ids[slot];
+    S.launched++;
+    return CRT_OK;
+}
+
+// Keeps the lanes fed: while the one with the fewest path ids ahead has less than two launches' worth,
+// the next segment in serving order goes to it. A short one (CRT_PATHS_MERGE) takes the whole of other
+// short requests of the same kernel along, one segment each, so that a queue of thumbnails fills the chip.
+int Context::launch_whole(const std::vector<ServeReq*>& act, bool& any_step) {
+    for (ServeReq* r : act)
+        if (!r->finishing && (r->cancel || r->job->scheduled_all())) {
+            int rc = finish_whole(0, r);
+            if (rc) return rc;
+            any_step = true;
+        }
+    for (;;) {
+        uint32_t lane = 0;
+        for (uint32_t l = 1; l < srv_lanes; ++l) if (srv[l].ids_ahead < srv[lane].ids_ahead) lane = l;
+        Server& S = srv[lane];
+        if (S.ids_ahead >= 2ull * kServeLaunch || S.launched - S.landed >= (uint64_t)Server::kRing) return CRT_OK;
+        const uint32_t cap = std::min(S.cap, kServeLaunch);
+        std::vector<std::pair<ServeReq*, WorkItem>> group;
+        uint32_t end = 0;
+        const uint32_t merge = (uint32_t)std::min<uint64_t>(
+            std::min(cap, CRT_PATHS_MERGE), S.gstack.bytes / sizeof(uint32_t) / crt_k_paths_overflow_entries());
+        for (ServeReq* r : serving_order(act, srv[0].rr)) {
+            if (r->finishing || r->job->scheduled_all()) continue;
+            Job& j = *r->job;
+            const bool stream = r->rd.rng_mode == CRT_RNG_MINSTD;
+            WorkItem w;
+            if (group.empty()) {
+                // MINSTD: a pixel's samples run in turn, so the launch is bounded by pixels and paths
+                const uint32_t c = !stream ? cap : std::min(cap, std::max(kServeStreams, kServeLaunch / std::max(1u, j.nsamples)));
+                if (!j.take_whole(c, w)) continue;
+            } else {
+                const uint64_t left = stream ? j.npix - j.p_next : j.paths_left();
+                w.job = &j;
+                if (!w.same_kernel(group[0].second) || whole_span(end) + left > merge) continue;
+                if (!j.take_whole(merge - whole_span(end), w)) continue;
+            }
+            end = whole_span(end) + w.whole_ids();
+            group.emplace_back(r, w);
+            if (whole_span(end) >= merge || group.size() >= Server::kLaunchEntries) break;
+        }
+        if (group.empty()) return CRT_OK;
+        any_step = true;
+        int rc = launch_group(lane, group);
+        if (rc) return rc;
+    }
+}
+
+// Takes finished launches off the lanes; `wait`: the one that the emptiest lane will finish next.
+int Context::land_launches(bool wait, bool& any_step) {
+    if (wait) {
+        int best = -1;
+        for (uint32_t l = 0; l < srv_lanes; ++l)
+            if (srv[l].landed < srv[l].launched && (best < 0 || srv[l].ids_ahead < srv[best].ids_ahead)) best = (int)l;
+        if (best >= 0) HIP_TRY(hipEventSynchronize(srv[best].ev[srv[best].landed % Server::kRing]));
+    }
+    for (uint32_t l = 0; l < srv_lanes; ++l) {
+        Server& S = srv[l];
+        while (S.landed < S.launched) {
+            const hipError_t q = hipEventQuery(S.ev[S.landed % Server::kRing]);
+            if (q == hipErrorNotReady) break;
+            HIP_TRY(q);
+            S.ids_ahead -= S.launch_ids[S.landed % Server::kRing];
+            S.landed++;
+            any_step = true;
+        }
+    }
+    return CRT_OK;
+}
+
+// Readback and completion of finished requests (completion thread; status != CRT_OK: no copies).
+void Context::server_complete(const std::vector<std::pair<ServeReq*, int>>& done) {
     Server& S = srv[0];   // owns the copy stream
-    if (st == CRT_OK) {
+    std::vector<HostStage::Copy> back;
+    std::vector<unsigned long long> rays(done.size(), 0);   // top bit: a whole-path launch ran out of traversal stack
+    for (size_t k = 0; k < done.size(); ++k) {
+        ServeReq* r = done[k].first;
+        if (done[k].second != CRT_OK) continue;
         // the accumulation buffer (16 B per pixel against 3 for the image) only when asked for
         const bool want_accum = !(r->rd.flags & CRT_RENDER_IMAGE_ONLY);
         r->rgb.resize((size_t)r->job->npix * 3);
         r->accum.resize(want_accum ? (size_t)r->job->npix * 4 : 0);
-        unsigned long long rays = 0;
-        const HostStage::Copy back[3] = {{&rays, r->job->rays_counter(), sizeof(rays)},
-                                         {r->rgb.data(), r->job->rgb.p, r->rgb.size()},
-                                         {r->accum.data(), r->job->accum.p, r->accum.size() * sizeof(float)}};
-        if (srv_stage.fetch(back, 3, S.copy_s) != hipSuccess)
-            st = set_error(CRT_ERR_HIP, "readback failed");
-        else
-            r->timing.rays = rays;
+        back.push_back({&rays[k], r->job->rays_counter(), sizeof(rays[k])});
+        back.push_back({r->rgb.data(), r->job->rgb.p, r->rgb.size()});
+        back.push_back({r->accum.data(), r->job->accum.p, r->accum.size() * sizeof(float)});
     }
-    if (r->ev_done) { (void)hipEventDestroy(r->ev_done); r->ev_done = nullptr; }
-    // the job's buffers go back to the cache (own lock); its stream work has completed
-    r->job.reset();
-    std::lock_guard<std::mutex> lk(srv_mutex);
-    request_bytes -= Job::bytes_needed(r->rd);
-    r->sc->refs--;
-    complete(r, st, srv_done_cv);
-    srv_cv.notify_all();   // the budget it held may admit a waiting request
+    const bool read = back.empty() || srv_stage.fetch(back.data(), (int)back.size(), S.copy_s) == hipSuccess;
+    for (size_t k = 0; k < done.size(); ++k) {
+        ServeReq* r = done[k].first;
+        int st = done[k].second;
+        if (st == CRT_OK) {
+            if (!read)
+                st = set_error(CRT_ERR_HIP, "readback failed");
+            else if (rays[k] >> 63)
+                st = set_error(CRT_ERR_INTERNAL, "traversal stack overflow");
+            else
+                r->timing.rays = rays[k];
+        }
+        if (r->ev_done) { (void)hipEventDestroy(r->ev_done); r->ev_done = nullptr; }
+        // the job's buffers go back to the cache (own lock); its stream work has completed
+        r->job.reset();
+        std::lock_guard<std::mutex> lk(srv_mutex);
+        request_bytes -= Job::bytes_needed(r->rd);
+        r->sc->refs--;
+        complete(r, st, srv_done_cv);
+        srv_cv.notify_all();   // the budget it held may admit a waiting request
+    }
 }
 
 void Context::server_copy_loop() {
     for (;;) {
-        std::pair<ServeReq*, int> job;
+        std::vector<std::pair<ServeReq*, int>> done;
         {
             std::unique_lock<std::mutex> lk(srv_mutex);
             srv_copy_cv.wait(lk, [&]() { return srv_copy_stop || !srv_copy_q.empty(); });
             if (srv_copy_q.empty()) return;   // stop requested and nothing left
-            job = srv_copy_q.front();
-            srv_copy_q.pop_front();
+            // small images that wait together are read back together
+            uint64_t bytes = 0;
+            do {
+                done.push_back(srv_copy_q.front());
+                srv_copy_q.pop_front();
+                bytes += Job::bytes_needed(done.back().first->rd);
+            } while (!srv_copy_q.empty() && bytes + Job::bytes_needed(srv_copy_q.front().first->rd) <= (8u << 20));
         }
-        server_complete(job.first, job.second);
+        server_complete(done);
     }
 }
 
@@ -481,7 +670,7 @@ void Context::server_loop() {
     }
     std::thread copier([this]() { server_copy_loop(); });
     auto lanes_inflight = [&]() {
-        for (uint32_t l = 0; l < L; ++l) if (srv[l].processed < srv[l].iter) return true;
+        for (uint32_t l = 0; l < L; ++l) if (srv[l].processed < srv[l].iter || srv[l].landed < srv[l].launched) return true;
         return false;
     };
     auto lanes_work = [&]() {
@@ -535,7 +724,7 @@ void Context::server_loop() {
             // (pinned by its reference) and the lane's own stream, so a blocking render holding
             // exec_mutex does not stall admission
             r->job = std::make_unique<Job>();
-            const int rc = r->job->setup(this, r->sc, r->rd, srv[r->lane].s);
+            const int rc = r->job->setup(this, r->sc, r->rd, srv[r->lane].s, serve_whole());
             r->timing.admit_s = now_s();
             std::lock_guard<std::mutex> lk(srv_mutex);
             if (rc) {
@@ -554,7 +743,14 @@ void Context::server_loop() {
         }
         bool busy = !admitted.empty(), any_step = false;
         std::vector<ServeReq*> lane_act[kSrvLanes];
-        for (uint32_t l = 0; l < L && !err; ++l) {
+        const bool whole = serve_whole();
+        if (whole) {
+            err = land_launches(false, any_step);
+            if (!err) err = launch_whole(act, any_step);
+            if (!err && !any_step) err = land_launches(true, any_step);
+            busy = busy || lanes_inflight();
+        }
+        for (uint32_t l = 0; l < L && !err && !whole; ++l) {
             Server& S = srv[l];
             std::vector<ServeReq*>& act_l = lane_act[l];
             for (ServeReq* r : act) if (r->lane == (int)l) act_l.push_back(r);
@@ -585,7 +781,7 @@ void Context::server_loop() {
             busy = busy || enqueued || S.processed < S.iter;
             any_step = any_step || enqueued || S.processed != processed0;
         }
-        if (!err && L > 1 && !any_step) {
+        if (!err && !whole && L > 1 && !any_step) {
             // nothing to launch and no finished iteration: wait for the oldest one in flight
             int oldest = -1;
             for (uint32_t l = 0; l < L; ++l)
@@ -620,6 +816,7 @@ void Context::server_loop() {
             for (uint32_t l = 0; l < L; ++l) {
                 (void)hipStreamSynchronize(srv[l].s);
                 srv[l].iter = srv[l].processed = 0;
+                srv[l].launched = srv[l].landed = srv[l].ids_ahead = 0;
                 server_reset_pass(srv[l]);
             }
             err = CRT_OK;
