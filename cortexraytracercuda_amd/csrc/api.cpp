@@ -815,9 +815,10 @@ int Context::run_whole(std::vector<WorkItem>& items, const PassBufs& B) {
     const uint32_t K = (uint32_t)std::min<size_t>(items.size(), std::min(sub_passes, B.max_sub));
     if (K > 1) HIP_TRY(hipEventRecord(ev_pass_ready, stream));
     for (uint32_t q = 1; q < K; ++q) HIP_TRY(hipStreamWaitEvent(sub_stream[q - 1], ev_pass_ready, 0));
-    // overflow stacks: an equal share of the allocation for each stream
-    const uint64_t wave_words = 64ull * crt_k_paths_overflow_entries();
-    const uint64_t waves = B.gstack_words / K / wave_words;
+    // overflow stacks and queues: an equal share of the allocation for each stream
+    const uint64_t words = B.gstack_words / K;
+    const uint32_t slots = B.slots / K;
+    const uint64_t waves = crt_k_paths_waves(words);
     if (waves == 0) return set_error(CRT_ERR_INTERNAL, "traversal stacks too small");
     uint32_t q = 0;
     for (size_t k = 0, m; k < items.size(); k = m, q = (q + 1) % K) {
@@ -831,9 +832,9 @@ int Context::run_whole(std::vector<WorkItem>& items, const PassBufs& B) {
         }
         hipStream_t s = q == 0 ? stream : sub_stream[q - 1];
         const HostScene& H = w.job->scene->host;
-        if (crt_k_paths(s, (int)w.job->rd.rng_mode, H.num_instances ? 1 : 0, H.num_shapes ? 1 : 0,
-                        (uint32_t)std::min<uint64_t>(waves, 1u << 20), (const crt_dev_scene*)scene_table.p, dreq + k,
-                        (uint32_t)(m - k), span, B.next + k, B.out_rad + host[k].path_base, B.gstack + q * waves * wave_words, B.counters))
+        if (crt_k_paths(s, (int)w.job->rd.rng_mode, H.num_instances ? 1 : 0, H.num_shapes ? 1 : 0, (uint32_t)H.num_node_records,
+                        (const crt_dev_scene*)scene_table.p, dreq + k, (uint32_t)(m - k), span, B.next + k, B.paths(0, q * slots),
+                        slots, B.out_rad + host[k].path_base, B.gstack + q * words, words, B.counters))
             return set_error(CRT_ERR_HIP, "path launch failed");
         if (w.job->rd.rng_mode == CRT_RNG_PCG && crt_k_resolve(s, dreq + k, (int)(m - k), max_pix, B.out_rad, nullptr))
             return set_error(CRT_ERR_HIP, "resolve launch failed");

@@ -113,6 +113,12 @@ __device__ __forceinline__ float4 ldg_at(const float4* base, uint32_t byte_off) 
     crt_v4f v = *(__attribute__((address_space(1))) const crt_v4f*)((gchar*)base + byte_off);
     return make_float4(v.x, v.y, v.z, v.w);
 }
+// The same with a constant byte offset behind it (the instruction's immediate).
+template <int IMM> __device__ __forceinline__ float4 ldg_off(const float4* base, uint32_t byte_off) {
+    typedef __attribute__((address_space(1))) const char gchar;
+    crt_v4f v = *(__attribute__((address_space(1))) const crt_v4f*)((gchar*)base + byte_off + (uint64_t)IMM);
+    return make_float4(v.x, v.y, v.z, v.w);
+}
 __device__ __forceinline__ int4 ldg_i4(const float4* p) {
     crt_v4i v = *(__attribute__((address_space(1))) const crt_v4i*)p;
     return make_int4(v.x, v.y, v.z, v.w);

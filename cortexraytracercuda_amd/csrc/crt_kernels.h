@@ -51,15 +51,16 @@ int crt_k_plain(hipStream_t s, int rng_mode, int width, int two_level, uint32_t 
                 const crt_dev_request* req, uint32_t* gstack, crt_dev_counters* counters);
 // Whole paths of `nreq` requests in one launch (paths.hip). `total` ids (pixels x samples, or pixels for
 // MINSTD, whose samples run in turn); `next` zeroed (nreq == 1); `out_rad` at the first request's
-// first id; `gstack` room for max_waves * 64 * crt_k_paths_overflow_entries() words. Several requests
+// first id; `gstack`: overflow stacks, for crt_k_paths_waves(gstack_words) waves. Several requests
 // share a launch when their ids, each request's from a path_base that is a multiple of
 // CRT_PATHS_ALIGN past the first one's, span at most CRT_PATHS_MERGE (`total` is that span) and
-// max_waves groups of CRT_PATHS_ALIGN.
+// as many groups of CRT_PATHS_ALIGN as there are such waves. `nodes`: the scene's node records, which
+// decide on refilled waves; their queues lie in the first `slots` entries of `queue`.
 constexpr uint32_t CRT_PATHS_ALIGN = 64u, CRT_PATHS_MERGE = 1u << 18;
-uint32_t crt_k_paths_overflow_entries(void);
-int crt_k_paths(hipStream_t s, int rng_mode, int two_level, int shapes, uint32_t max_waves, const crt_dev_scene* scenes,
-                const crt_dev_request* reqs, uint32_t nreq, uint32_t total, uint32_t* next, float4* out_rad, uint32_t* gstack,
-                crt_dev_counters* counters);
+uint32_t crt_k_paths_waves(uint64_t gstack_words);
+int crt_k_paths(hipStream_t s, int rng_mode, int two_level, int shapes, uint32_t nodes, const crt_dev_scene* scenes,
+                const crt_dev_request* reqs, uint32_t nreq, uint32_t total, uint32_t* next, crt_paths queue, uint32_t slots,
+                float4* out_rad, uint32_t* gstack, uint64_t gstack_words, crt_dev_counters* counters);
 // Closest hits of n rays into `out`: n primitive ids, n instance ids, n distances, n (u, v) pairs.
 int crt_k_trace_rays(hipStream_t s, int width, int two_level, uint32_t grid, const crt_dev_scene* sc, const float4* rays,
                      uint32_t n, int camera, uint32_t* out, uint32_t* gstack, crt_dev_counters* counters);

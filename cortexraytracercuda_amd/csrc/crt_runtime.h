@@ -284,8 +284,9 @@ struct Context {
     // up to kSrvLanes open passes on their own streams (each with a share of the slot pool), so one
     // pass's drain tail overlaps the other's full launches; a request's segments stay in one lane
     static constexpr int kSrvLanes = 2;
-    // path ids of one whole-path launch of the serving loop
-    static constexpr uint32_t kServeLaunch = 1u << 22, kServeStreams = 1u << 18;
+    // path ids of one whole-path launch of the serving loop, at least for MINSTD, whose ids are pixels;
+    // a lane with kServeAhead of them gets no more
+    static constexpr uint32_t kServeLaunch = 1u << 23, kServeStreams = 1u << 18, kServeAhead = 1u << 23;
     Server srv[kSrvLanes];
     uint32_t srv_lanes = 1;
     uint64_t lane_load[kSrvLanes] = {};

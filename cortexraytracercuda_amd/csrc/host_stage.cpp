@@ -77,7 +77,7 @@ hipError_t HostStage::fetch(const Copy* list, int n, hipStream_t s) {
         return hipSuccess;
     }
     // pieces of at most a chunk; short ones share a slot (a slot's event and its wait cost more than the
-    // copies of an image of 64x64: 64 of them with their sums, 3.1 -> STAGE_AFTER ms for the whole call)
+    // copy of a 64x64 image)
     std::vector<Piece> pieces;
     std::vector<size_t> first;   // first piece of each slotful
     size_t room = 0;

@@ -6,14 +6,15 @@
 //   - requests are admitted first-fit against the HBM budget (accumulation, tonemap and RNG
 //     buffers; scenes are already resident and counted at upload) and join the lane with the
 //     fewest outstanding paths;
-//   - an admitted request is cut into segments (pixel range x sample range) of up to 4 M paths; a
+//   - an admitted request is cut into segments (pixel range x sample range) of up to 8 M paths; a
 //     segment is one launch that follows its paths to their end, and its resolve, on the lane with
-//     the fewest paths ahead; the next ones are enqueued while fewer than two launches' worth are.
+//     the fewest paths ahead; the next ones are enqueued while fewer than 8 M are.
 //     Segments of one request are resolved in sample order by events between the lanes; after the
 //     last one comes the tonemap, and a completion thread reads the image back;
 //   - short segments of several requests share a launch.
 // One request's paths no longer wait for the others' between bounces as in the iterations below, and
-// their state stays off HBM: SERVE_FIGURES.
+// their state stays off HBM: 20 queued requests on four scenes 323 -> 214 ms, a 64x64 request behind two of
+// 1024x1024 at 64 samples 171 -> 24 ms, one of those alone 106 -> 66 ms.
 // Contexts whose renders run in stages (two-wide nodes, a closest-hit stage asked for) serve in stages:
 //   - a segment becomes a request-table entry of its lane's open pass and its path ids are appended
 //     behind the pass's last id between two iterations, so the next regeneration stage already starts
@@ -504,13 +505,15 @@ int Context::launch_group(uint32_t lane, std::vector<std::pair<ServeReq*, WorkIt
     if (end > S.cap) return set_error(CRT_ERR_INTERNAL, "launch exceeds the lane's path ids");
     const WorkItem& w0 = group[0].second;
     const HostScene& H = w0.job->scene->host;
-    const uint64_t waves = S.gstack.bytes / sizeof(uint32_t) / (64ull * crt_k_paths_overflow_entries());
     uint32_t* next = (uint32_t*)S.live_min.p;
     HIP_TRY(hipMemcpyAsync(dreq, S.req_host + e0, sizeof(crt_dev_request) * group.size(), hipMemcpyHostToDevice, S.s));
     if (crt_k_fill_u32(S.s, next, 1u, 0u)) return set_error(CRT_ERR_HIP, "fill launch failed");
-    if (crt_k_paths(S.s, (int)w0.job->rd.rng_mode, H.num_instances ? 1 : 0, H.num_shapes ? 1 : 0,
-                    (uint32_t)std::min<uint64_t>(waves, 1u << 20), (const crt_dev_scene*)scene_table.p, dreq,
-                    (uint32_t)group.size(), end, next, (float4*)S.out_rad.p, (uint32_t*)S.gstack.p, (crt_dev_counters*)S.counters.p))
+    crt_paths queue;
+    queue.ray_o = (float4*)S.ray_o[0].p; queue.ray_d = (float4*)S.ray_d[0].p; queue.thr = (float4*)S.thr[0].p;
+    queue.rad = (float4*)S.rad[0].p; queue.ids = (uint2*)S.ids[0].p;
+    if (crt_k_paths(S.s, (int)w0.job->rd.rng_mode, H.num_instances ? 1 : 0, H.num_shapes ? 1 : 0, (uint32_t)H.num_node_records,
+                    (const crt_dev_scene*)scene_table.p, dreq, (uint32_t)group.size(), end, next, queue, S.slots,
+                    (float4*)S.out_rad.p, (uint32_t*)S.gstack.p, S.gstack.bytes / sizeof(uint32_t), (crt_dev_counters*)S.counters.p))
         return set_error(CRT_ERR_HIP, "path launch failed");
     if (w0.job->rd.rng_mode == CRT_RNG_PCG) {
         // segments of one request are resolved in sample order, whichever lanes traced them
@@ -535,9 +538,11 @@ int Context::launch_group(uint32_t lane, std::vector<std::pair<ServeReq*, WorkIt
     return CRT_OK;
 }
 
-// Keeps the lanes fed: while the one with the fewest path ids ahead has less than two launches' worth,
-// the next segment in serving order goes to it. A short one (CRT_PATHS_MERGE) takes the whole of other
-// short requests of the same kernel along, one segment each, so that a queue of thumbnails fills the chip.
+// Keeps the lanes fed: while the one with the fewest path ids ahead has less than kServeAhead, the next
+// segment in serving order goes to it. A short one (CRT_PATHS_MERGE) takes the whole of other short
+// requests of the same kernel along, so that a queue of thumbnails fills the chip. Launches of 1, 4, 8 and
+// 16 M paths: 290, 221, 214 and 209 ms for 20 requests; the more, the longer a small request waits (7, 22,
+// 24 and 76 ms behind two large ones).
 int Context::launch_whole(const std::vector<ServeReq*>& act, bool& any_step) {
     for (ServeReq* r : act)
         if (!r->finishing && (r->cancel || r->job->scheduled_all())) {
@@ -549,12 +554,12 @@ int Context::launch_whole(const std::vector<ServeReq*>& act, bool& any_step) {
         uint32_t lane = 0;
         for (uint32_t l = 1; l < srv_lanes; ++l) if (srv[l].ids_ahead < srv[lane].ids_ahead) lane = l;
         Server& S = srv[lane];
-        if (S.ids_ahead >= 2ull * kServeLaunch || S.launched - S.landed >= (uint64_t)Server::kRing) return CRT_OK;
+        if (S.ids_ahead >= kServeAhead || S.launched - S.landed >= (uint64_t)Server::kRing) return CRT_OK;
         const uint32_t cap = std::min(S.cap, kServeLaunch);
         std::vector<std::pair<ServeReq*, WorkItem>> group;
         uint32_t end = 0;
         const uint32_t merge = (uint32_t)std::min<uint64_t>(
-            std::min(cap, CRT_PATHS_MERGE), S.gstack.bytes / sizeof(uint32_t) / crt_k_paths_overflow_entries());
+            std::min(cap, CRT_PATHS_MERGE), (uint64_t)CRT_PATHS_ALIGN * crt_k_paths_waves(S.gstack.bytes / sizeof(uint32_t)));
         for (ServeReq* r : serving_order(act, srv[0].rr)) {
             if (r->finishing || r->job->scheduled_all()) continue;
             Job& j = *r->job;

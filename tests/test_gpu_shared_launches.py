@@ -39,7 +39,7 @@ def test_short_requests_of_several_scenes(rng):
 
 @pytest.mark.parametrize("paths", [1 << 20, 3000])
 def test_long_requests_over_both_lanes_among_short_ones(paths):
-    """Requests of several segments (4 M paths; 1,500 ids a lane in the small pool), cancelled ones between."""
+    """Requests of several segments (8 M paths; 1,500 ids a lane in the small pool), cancelled ones between."""
     big = (1200, 900, 9) if paths > 3000 else (90, 40, 4)
     with Renderer(max_paths=paths, pass_paths=0 if paths > 3000 else paths) as r:
         sid = r.upload(scenes.sphere_mesh_scene(20000, seed=4))
