@@ -6,12 +6,12 @@ streams, seed 1. One step = one complete render of that image (every sample of e
 
 Printed JSON line (rank 0):
   value        Mrays/s over the timed steps (closest-hit queries / wall time of the renders)
-  roofline     traversal kernel (k_extend) against its binding resource, VALU issue: VALU wave
-               instructions per ray (rocprofv3 SQ counters, profiles/) x rays per launch / HIP-event
-               launch time, against 1024 SIMDs x 2.4 GHz / 4 cycles per wave64 instruction (dense
-               FMA-class issue; the measured probe rates of profiles/valu_issue_probe_mi355x.json
-               beside it); with the measured DRAM traffic (FETCH_SIZE / WRITE_SIZE) and the
-               algorithmic bytes
+  roofline     the kernel that follows the paths (k_paths_refill / k_paths; k_extend where the render
+               runs in stages) against its binding resource, VALU issue: VALU wave instructions per
+               ray (rocprofv3 SQ counters, profiles/) x rays per launch / HIP-event time, against 1024
+               SIMDs x 2.4 GHz / 4 cycles per wave64 instruction (dense FMA-class issue; the measured
+               probe rates of profiles/valu_issue_probe_mi355x.json beside it); with the measured DRAM
+               traffic (FETCH_SIZE / WRITE_SIZE) and the algorithmic bytes
   cpu_baseline reference-faithful CPU renderer (oracle/, FP32 minstd) on the host cores, 4 spp,
                plus a one-thread figure and the host CPU model
   megakernel   the plain path on the same workload: one kernel launch renders the image
@@ -44,7 +44,8 @@ VALU_PEAK_GINST = 1024 * 2.4 / 4.0
 #   + 64 B per BVH2 / 128 B per BVH4 interior node visit (child boxes + refs; a leaf's type, count
 #   and first primitive are packed into its reference in the parent, so a leaf visit reads nothing),
 #   + 48 B per triangle, 16 B per sphere, 80 B per quad/light, 64 B per instance record.
-B_STATE = 64
+# A whole-path launch keeps a path's state on chip: 16 B of radiance per path.
+B_STATE, B_PATH = 64, 16
 B_LEAF, B_TRI, B_SPHERE, B_QUAD, B_INST = 0, 48, 16, 80, 64   # node bytes come from the scene (64 or 128)
 
 
@@ -242,12 +243,17 @@ def serving(seed=11, n=48, rate_hz=60.0):
     return out
 
 
-def _profile_json(kind, workload_key, inf):
-    """A committed counter summary (profiles/k_extend_<kind>_<workload>.json) for the BVH shape
+def _runs_whole(args, inf):
+    """Renders follow whole paths in one launch unless the closest-hit stage or two-wide nodes are asked for."""
+    return not args.extend_kernel and inf["bvh_width"] == 4
+
+
+def _profile_json(kernel, kind, workload_key, inf):
+    """A committed counter summary (profiles/<kernel>_<kind>_<workload>.json) for the BVH shape
     it was taken on, or None."""
     if not workload_key:
         return None
-    path = os.path.join(ROOT, "profiles", "k_extend_%s_%s.json" % (kind, workload_key))
+    path = os.path.join(ROOT, "profiles", "%s_%s_%s.json" % (kernel, kind, workload_key))
     if not os.path.exists(path):
         return None
     with open(path) as f:
@@ -258,8 +264,9 @@ def _profile_json(kind, workload_key, inf):
 
 
 def traversal_roofline(scene, cfg, args, timed_renderer, sid, progressive=False, workload_key=""):
-    """k_extend roofline for one render of the workload. The launches are timed with HIP events on
-    their stream. The binding resource is VALU issue: VALU wave instructions per ray (SQ_INSTS_VALU
+    """Roofline of the path kernel (of k_extend where the render runs in stages) for one render of the
+    workload. The launches are timed with HIP events on their stream; a whole-path launch with the
+    resolve behind it (0.4 of 20 ms at 1080p, 64 spp). The binding resource is VALU issue: VALU wave instructions per ray (SQ_INSTS_VALU
     of the same kernel on the same workload, profiles/) times the rays of a launch over its time,
     against VALU_PEAK_GINST. Beside it: DRAM bytes per launch (FETCH_SIZE / WRITE_SIZE, profiles/)
     and the algorithmic bytes (node and primitive records of every visit, from the counting variant
@@ -274,7 +281,8 @@ def traversal_roofline(scene, cfg, args, timed_renderer, sid, progressive=False,
     node_b = inf["node_bytes"]
     cnt = dict.fromkeys(["rays", "node_visits", "leaf_visits", "tri_tests", "sphere_tests", "quad_tests", "inst_visits"], 0)
     ext_ms = 0.0
-    launches = 0
+    launches = paths = 0
+    whole = _runs_whole(args, inf)
     ranges = [(k, 1) for k in range(cfg["spp"])] if progressive else [(0, 0)]
     for sb, sc in ranges:
         rc.render(sidc, cfg["width"], cfg["height"], cfg["spp"], cfg["max_depth"], seed=1, sample_begin=sb,
@@ -283,25 +291,27 @@ def traversal_roofline(scene, cfg, args, timed_renderer, sid, progressive=False,
         for k in cnt:
             cnt[k] += c[k]
         _, _, stt = timed_renderer.render(sid, cfg["width"], cfg["height"], cfg["spp"], cfg["max_depth"], seed=1,
-                                          sample_begin=sb, sample_count=sc, want_accum=False, time_stages=True)
-        ext_ms += stt["extend_ms"]
-        launches += timed_renderer.extend_launches()
+                                          sample_begin=sb, sample_count=sc, want_accum=False, time_stages=not whole)
+        ext_ms += stt["gpu_ms" if whole else "extend_ms"]
+        launches += 1 if whole else timed_renderer.extend_launches()
+        paths += stt["paths"]
     rc.close()
-    alg = (B_STATE * cnt["rays"] + node_b * cnt["node_visits"] + B_LEAF * cnt["leaf_visits"] + B_TRI * cnt["tri_tests"] +
+    alg = ((B_PATH * paths if whole else B_STATE * cnt["rays"]) + node_b * cnt["node_visits"] + B_LEAF * cnt["leaf_visits"] + B_TRI * cnt["tri_tests"] +
            B_SPHERE * cnt["sphere_tests"] + B_QUAD * cnt["quad_tests"] + B_INST * cnt["inst_visits"])
     launches = max(launches, 1)
     launch_s = ext_ms / launches * 1e-3
     rays_per_launch = cnt["rays"] / launches
     algorithmic_gbs = alg / (ext_ms * 1e-3) / 1e9
+    kernel = "k_paths" if whole else "k_extend"
     # measured DRAM bytes (rocprofv3 FETCH_SIZE / WRITE_SIZE, scaled by a 1 GiB copy) per ray of this
-    # workload's closest-hit kernel, times the rays of one launch; null for workloads not profiled
-    tr = _profile_json("traffic", workload_key, inf)
+    # workload's kernel, times the rays of one launch; null for workloads not profiled
+    tr = _profile_json(kernel, "traffic", workload_key, inf)
     traffic = None if tr is None else tr["hbm_bytes_per_ray"] * rays_per_launch
     dram = None if traffic is None else traffic / launch_s / 1e9
-    sq = _profile_json("sq", workload_key, inf)
+    sq = _profile_json(kernel, "sq", workload_key, inf)
     probe_path = os.path.join(ROOT, "profiles", "valu_issue_probe_mi355x.json")
     probe = json.load(open(probe_path))["rates_ginst_s"] if os.path.exists(probe_path) else {}
-    roof = {"kernel": "k_extend", "launches": launches, "avg_launch_ms": ext_ms / launches,
+    roof = {"kernel": kernel if sq is None else sq["kernel"], "launches": launches, "avg_launch_ms": ext_ms / launches,
             "rays_per_launch": rays_per_launch,
             "traffic": traffic, "traffic_unit": "bytes per launch",
             "dram_gbs": dram, "dram_frac": None if dram is None else dram / HBM_PEAK_GBS,
@@ -443,8 +453,8 @@ def valu_probe(iters=100000):
 
 def one_render_probe(scene, cfg, args, progressive):
     """One render of the workload with the library's default shape, in the form the roofline times
-    (stages timed with HIP events: one sub-pass, the launches of traversal_roofline; no counting
-    variant): the rays and kernel launches a counter run divides its per-dispatch sums by."""
+    (whole-path launches, or stages timed with HIP events: the launches of traversal_roofline; no
+    counting variant): the rays and kernel launches a counter run divides its per-dispatch sums by."""
     from cortexraytracercuda_amd import Renderer
     r = Renderer(bvh_width=args.bvh_width, max_paths=args.max_paths, extend_kernel=args.extend_kernel,
                  refill_min=args.refill_min, grid_per_cu=args.grid_per_cu, shade_grid_per_cu=args.shade_grid_per_cu,
@@ -453,12 +463,13 @@ def one_render_probe(scene, cfg, args, progressive):
     info = r.info(sid)
     ranges = [(k, 1) for k in range(cfg["spp"])] if progressive else [(0, 0)]
     rays = launches = exact = 0
+    whole = _runs_whole(args, info)
     for sb, sc in ranges:
         _, _, st = r.render(sid, cfg["width"], cfg["height"], cfg["spp"], cfg["max_depth"], seed=1, sample_begin=sb,
-                            sample_count=sc, want_accum=False, time_stages=True)
+                            sample_count=sc, want_accum=False, time_stages=not whole)
         c = r.counters()
         rays += st["rays"]
-        launches += c["extend_launches"]
+        launches += 1 if whole else c["extend_launches"]
         exact += c["exact_queries"]
     r.close()
     return {"one_render": True, "config": cfg, "passes": len(ranges), "rays": rays, "extend_launches": launches,

@@ -145,10 +145,10 @@ struct ServeReq {
     crt_request_timing timing{};
     int status = CRT_ERR_NOT_READY;
     bool cancel = false;
-    uint32_t segs = 0;             // segments appended to the open pass
+    uint32_t segs = 0;             // segments launched, or appended to the open pass
     uint32_t segs_resolved = 0;    // segments whose resolve has been enqueued (in segment order)
     bool finishing = false;        // tonemap + readback enqueued, waiting for ev_done
-    int lane = 0;                  // open pass (server lane) that traces all of its segments
+    int lane = 0;                  // stages: the open pass (server lane) that traces all of its segments
     uint64_t load = 0;             // paths it adds to its lane's load until it completes
     hipEvent_t ev_done = nullptr;
     // whole-path launches: the lanes that have its buffers' start behind them, and the number (from 1)

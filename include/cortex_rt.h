@@ -331,8 +331,8 @@ typedef struct crt_config {
     uint32_t grid_per_cu;       /* workgroups per CU of the closest-hit launches (256 threads each); 0 = 24 */
     uint32_t shade_grid_per_cu; /* workgroups per CU of the regenerate / shade launches; 0 = 16 */
     uint32_t sub_passes;        /* concurrent sub-passes (one stream each) of a pass, 1-4; 0 = 2 */
-    uint32_t graphs;            /* serving loop iterations replayed from hipGraphs: 0 = default (on), 1 = on,
-                                   2 = off (every iteration launched eagerly) */
+    uint32_t graphs;            /* iterations of a serving loop that runs in stages replayed from hipGraphs:
+                                   0 = default (on), 1 = on, 2 = off (every iteration launched eagerly) */
     uint32_t stack_lds;         /* traversal stack: LDS ring entries per lane behind the register top entry,
                                    8, 16 or 32; 0 = 16 */
     uint32_t ray_sort;          /* 1: the shade stage groups each workgroup's surviving paths by direction

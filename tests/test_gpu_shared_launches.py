@@ -50,3 +50,17 @@ def test_long_requests_over_both_lanes_among_short_ones(paths):
         r.cancel(dropped)
         got = [r.wait(i, j["width"], j["height"]) for i, j in zip(ids, jobs)]
         _check(r, jobs, [(rgb, acc, st["rays"]) for rgb, acc, st in got])
+
+
+@pytest.mark.parametrize("config", [dict(extend_kernel=1, graphs=1), dict(extend_kernel=1, graphs=2), dict(bvh_width=2)])
+def test_contexts_that_run_in_stages_serve_in_stages(config):
+    """The open passes of the stages (enough iterations that captured ones are replayed) give what
+    whole-path launches give."""
+    s = scenes.sphere_mesh_scene(5000, seed=1)
+    with Renderer(max_paths=1 << 16, pass_paths=1 << 18) as whole, Renderer(max_paths=1 << 16, pass_paths=1 << 18, **config) as r:
+        a, b = whole.upload(s), r.upload(s)
+        jobs = [dict(width=97, height=61, spp=9, max_depth=6, seed=k, rng=m) for k, m in enumerate(["pcg", "minstd", "pcg", "pcg"])]
+        for _ in range(3):
+            ids = [r.submit(b, **j) for j in jobs]
+            got = [r.wait(i, j["width"], j["height"]) for i, j in zip(ids, jobs)]
+            _check(whole, [dict(j, sid=a) for j in jobs], [(rgb, acc, st["rays"]) for rgb, acc, st in got])
