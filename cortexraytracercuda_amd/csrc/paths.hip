@@ -242,9 +242,10 @@ constexpr uint32_t kRefill = 40, kLeafShare = 4, kDrainLive = 56, kQueueShare = 
 // 5.0 -> 5.3, 33,066: 5.5 -> 5.7 (1080p 49 spp: 13.0 -> 13.2), 132,139: 6.1 -> 6.2, 526,438: 6.8 -> 6.7. By paths, room of 78,322 and open scene of 132,139 nodes: 4 M 4.46 -> 4.22 and 1.56 -> 1.71, 9 M 9.5 ->
 // 8.6 and 2.4 -> 2.5, 16 M 16.1 -> 14.0 and 3.47 -> 3.49.
 constexpr uint32_t kRefillNodes = 1u << 14, kRefillPaths = 3u << 21;
-// Stack entries of a lane in global memory: the ring's entries have their place there too (8 + 104 entries
-// as in k_paths, 3 that one node may push beyond) and the last holds the start of a re-traced ray.
-constexpr int kRefillStack = kLds + kOverflow + 4;
+// Stack entries of a lane in global memory: the ring's entries have their place there too (as many in
+// all as k_paths has with its register entry, 113, and more), three that one node may push beyond, and
+// the last one holds the start of a re-traced ray. The state word counts them in 7 bits.
+constexpr int kRefillStack = kLds + kOverflow + 8;
 
 // Box tests are accepted up to this multiple of the closest distance so far (the tie window, and the
 // box test's own rounding).
