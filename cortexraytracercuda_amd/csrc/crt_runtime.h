@@ -220,7 +220,7 @@ struct Context {
     int extend_mode = CRT_EXTEND_GRID_STRIDE;   // closest-hit work distribution (CRT_EXTEND_*)
     uint32_t extend_param = 2;       // lane-refill threshold or 64-ray groups per wave fetch
     uint32_t stack_lds = 16;         // LDS ring entries per lane of the traversal stack (8, 16, 32)
-    bool staged = false;             // blocking renders run as stage launches (asked for by extend_kernel, ray_sort or count_work)
+    bool staged = false;             // renders run as stage launches (asked for by extend_kernel, ray_sort or count_work)
     uint32_t ray_sort = 0;           // shade groups each block's survivors by direction octant
     uint32_t bvh_builder = CRT_BVH_HOST;   // where crt_scene_upload builds the BVH (CRT_BVH_*)
     uint64_t batch_group = 1ull << 22;     // path ids left for a batched request to get passes of its own scene

@@ -32,9 +32,10 @@ __device__ __forceinline__ uint32_t lane_rank(uint64_t mask) {
     return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
 }
 
-// Follows the paths of one request (ids [0, total): its pixels, each pixel's samples consecutive), or of
-// several short ones, to their end in one launch. A workgroup is one wave. Each round the wave holds at most `group` paths,
-// one per lane, and traces and shades one segment of each:
+// Follows the paths of one request (ids [0, total): its pixels, each pixel's samples consecutive) to
+// their end in one launch; MERGED, of several short ones (a branch for both in one kernel costs the
+// two-level loop 8 %, in registers). A workgroup is one wave. Each round the wave holds at most `group`
+// paths, one per lane, and traces and shades one segment of each:
 //   - lanes whose path ended take a path from the wave's queue in LDS;
 //   - when queue and live paths together no longer fill a group, the live ones are put in the queue
 //     (it never holds a whole group) and the next `group` ids start at the camera, so camera rays stay
@@ -45,8 +46,8 @@ __device__ __forceinline__ uint32_t lane_rank(uint64_t mask) {
 // and a launch whose last wave the next one waits for on each bounce. Here a path's state stays in
 // registers and LDS, and only its radiance (16 B) is written. What bounds it is the traversal's VALU
 // issue. Staged against this, GPU time of one render: 1080p 64 spp large scene 31.5 -> 20.8 ms,
-// 2M-triangle room 1024^2 64 spp 81.2 -> 68.5, shapes 640x360 16 spp 4.8 -> 1.25 (latency and tails of
-// the 22 launch rounds), box 64^2 16 spp 0.50 -> 0.17; 4,096 instances 4K 1 spp 27.0 -> 26.6.
+// 2M-triangle room 1024^2 64 spp 80.6 -> 67.1, shapes 640x360 16 spp 4.8 -> 1.25 (latency and tails of
+// the 22 launch rounds), box 64^2 16 spp 0.50 -> 0.17; 4,096 instances 4K 1 spp 27.0 -> 24.2.
 // MINSTD: an id is a pixel; its samples run one after the other in its lane, each ended path starting
 // the next sample, and are added to the accumulation buffer in order (a scene file's 512x388, 49
 // samples, depth 100: 61 -> 5.7 ms against one staged pass per sample).

@@ -2,10 +2,9 @@
 //
 // The reference serves one render per process (UI/Examples/UI/main.cpp:371-395 spawns the exe)
 // with no queue, batching or residency. Here one scheduler thread owns streams and path pools of
-// its own and keeps one streaming pass open per lane (two lanes, each with half the slots):
+// its own, on two lanes (streams with half the slots each):
 //   - requests are admitted first-fit against the HBM budget (accumulation, tonemap and RNG
-//     buffers; scenes are already resident and counted at upload) and join the lane with the
-//     fewest outstanding paths;
+//     buffers; scenes are already resident and counted at upload);
 //   - an admitted request is cut into segments (pixel range x sample range) of up to 8 M paths; a
 //     segment is one launch that follows its paths to their end, and its resolve, on the lane with
 //     the fewest paths ahead; the next ones are enqueued while fewer than 8 M are.
@@ -16,6 +15,7 @@
 // their state stays off HBM: 20 queued requests on four scenes 323 -> 214 ms, a 64x64 request behind two of
 // 1024x1024 at 64 samples 171 -> 24 ms, one of those alone 106 -> 66 ms.
 // Contexts whose renders run in stages (two-wide nodes, a closest-hit stage asked for) serve in stages:
+//   - an admitted request joins the lane with the fewest outstanding paths; each lane keeps one pass open;
 //   - a segment becomes a request-table entry of its lane's open pass and its path ids are appended
 //     behind the pass's last id between two iterations, so the next regeneration stage already starts
 //     its camera rays among the paths of every other request in flight;

@@ -315,10 +315,10 @@ typedef struct crt_config {
     uint32_t count_work;        /* 1: use the counting traversal kernel (fills node_visits/prim_tests) */
     uint32_t leaf_size;         /* BVH max primitives per leaf (1-8); 0 = default (1) */
     uint32_t bvh_width;         /* children per BVH node, 2 or 4; 0 = default (4) */
-    uint32_t extend_kernel;     /* 0 = default: blocking renders of four-wide scenes follow whole paths in one
-                                   launch per request; where stages run all the same (two-wide scenes, the
-                                   serving loop, CRT_RENDER_TIME_STAGES, count_work), as with 1. Otherwise
-                                   every render runs in stages, with this closest-hit stage (CRT_EXTEND_*):
+    uint32_t extend_kernel;     /* 0 = default: renders and served requests of four-wide scenes follow whole
+                                   paths in one launch per request or segment; where stages run all the same
+                                   (two-wide scenes, CRT_RENDER_TIME_STAGES, count_work), as with 1. Otherwise
+                                   everything runs in stages, with this closest-hit stage (CRT_EXTEND_*):
                                    1 = grid-stride (each lane
                                    traces its rays to the end, the wave waits for its slowest lane),
                                    2 = per-lane refill: a lane whose ray is done takes the next ray of its
