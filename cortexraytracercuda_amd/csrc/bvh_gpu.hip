@@ -497,6 +497,14 @@ int gpu_build_scene(Context& C, const crt_scene_desc* d, uint32_t leaf, uint32_t
     Context* ctx = &C;
     // source records on the device
     DevBuf squads, sqbox, ssph, stris, snrm, suv, smap;
+    // work buffers
+    DevBuf plo, phi, keys[2], vals[2], cb, cl, cr, nlo, nhi, first, count, tmask, tflags, ranks, slot_b, level_base,
+        counters, sah, nodes_tmp, tmp, srcmap;
+    std::vector<uint32_t> lb, srch;   // read back
+    struct Drain {   // behind every buffer: none goes back while work on it is still queued, on error returns as well
+        hipStream_t s;
+        ~Drain() { (void)hipStreamSynchronize(s); }
+    } drain{s};
     // work buffers come from and return to the context's cache (an allocation and its free cost 0.1-0.4 ms
     // each, and a build takes thirty); large ones at their own size (the cache's classes are powers of two)
     auto work = [&](DevBuf& b, size_t bytes) { return bytes <= (256ull << 20) ? b.alloc_cached(bytes, ctx) : b.alloc(bytes, ctx); };
@@ -516,13 +524,6 @@ int gpu_build_scene(Context& C, const crt_scene_desc* d, uint32_t leaf, uint32_t
     if ((rc = up(suv, src.tri_uvs.data(), src.tri_uvs.size() * sizeof(F2)))) return rc;
     Prims P{dptr<float4>(squads), dptr<float4>(sqbox), dptr<float4>(ssph), dptr<float4>(stris), nq, ns, nt};
 
-    // work buffers
-    DevBuf plo, phi, keys[2], vals[2], cb, cl, cr, nlo, nhi, first, count, tmask, tflags, ranks, slot_b, level_base,
-        counters, sah, nodes_tmp, tmp, srcmap;
-    struct Drain {   // no buffer goes back while work on it is still queued, on error returns as well
-        hipStream_t s;
-        ~Drain() { (void)hipStreamSynchronize(s); }
-    } drain{s};
     RangeLevels RL{};
     uint64_t rn = 0;
     for (uint64_t m = n; RL.levels < RangeLevels::kMax; m = (m + 1) / 2) {
@@ -598,7 +599,7 @@ int gpu_build_scene(Context& C, const crt_scene_desc* d, uint32_t leaf, uint32_t
            dptr<uint32_t>(count), dptr<uint32_t>(tmask), svals, dptr<float4>(plo), dptr<float4>(phi), dptr<TypeCount>(ranks),
            P, std::max(1u, std::min(leaf, CRT_LEAF_MAX_COUNT))};
     // 6. collapse, level by level; the level bases are read back every few levels to stop
-    std::vector<uint32_t> lb(kMaxLevels + 2, 0);
+    lb.assign(kMaxLevels + 2, 0);
     int levels = 0;
     const uint32_t cgrid = grid_for(n / 2 + 1, 2048);
     for (int L = 0; L < kMaxLevels; ++L) {
@@ -655,7 +656,7 @@ int gpu_build_scene(Context& C, const crt_scene_desc* d, uint32_t leaf, uint32_t
                                  (float4*)(geo + tri_off), (float4*)(geo + sph_off), (float4*)(geo + quad_off),
                                  dptr<float4>(sc.tri_normals), dptr<float2>(sc.tri_uvs), dptr<float2>(sc.sphere_map),
                                  src_tri, src_sph, src_quad), "scatter");
-    std::vector<uint32_t> srch((size_t)nt + ns + nq);
+    srch.resize((size_t)nt + ns + nq);
     const HostStage::Copy back{srch.data(), srcmap.p, srch.size() * 4};
     HIP_TRY(ctx->stage.fetch(&back, 1, s));
     if ((rc = (sc.mats.alloc(H.mats.size() * 16, ctx)))) return rc;

@@ -1,0 +1,23 @@
+"""Calls that fail half way leave no queued work behind that names their buffers: those go back to a cache
+that other streams take from. On the CPU (hip_standin)."""
+import numpy as np
+import pytest
+
+from cortexraytracercuda_amd import Renderer, _abi as A, scenes
+from hip_standin import standin, standin_lib  # noqa: F401
+
+
+@pytest.mark.parametrize("normals", [False, True])
+def test_a_device_build_that_fails_leaves_nothing_queued(standin, normals):
+    s = scenes.sphere_mesh_scene(3000, seed=1)
+    s.sphere((0.1, 0.2, 0.3), 0.2, s.lambertian(None, (0.5, 0.5, 0.5)))
+    if normals:
+        m = s.meshes[0]
+        m["normals"] = np.ones_like(m["positions"])
+    with Renderer(max_paths=4096, pass_paths=4096, bvh_builder="device") as r:
+        # one source buffer after the other: those before it come from the cache, all but the last one
+        for n in range(5 + normals):
+            r.lib.crt_debug_fail_alloc(r.h, min(n, 1))
+            with pytest.raises(A.CrtError, match="injected"):
+                r.upload(s)
+            assert standin.standin_pending() == 0, n
