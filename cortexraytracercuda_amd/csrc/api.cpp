@@ -1163,7 +1163,9 @@ int crt_trace_rays(crt_context* c, crt_scene_id s, const float* rays, uint64_t n
     // per-call buffers from the context's cache; large ones at their own size (the cache's classes are
     // powers of two)
     auto get = [&](DevBuf& b, uint64_t bytes) { return bytes <= (256ull << 20) ? b.alloc_cached(bytes, ctx) : b.alloc(bytes, ctx); };
-    DevBuf out;
+    DevBuf out, dr, dh, di, dro, drd, dids, dctl;
+    std::vector<float> po, pd;
+    const StreamDrain drain(ctx->stream);
     int rc;
     const bool camera = (flags & CRT_TRACE_CAMERA) != 0;
     if ((rc = get(out, n * 20))) return rc;
@@ -1171,8 +1173,6 @@ int crt_trace_rays(crt_context* c, crt_scene_id s, const float* rays, uint64_t n
     uint32_t grid = std::min(ctx->extend_grid, (uint32_t)std::max<uint64_t>(1, (n + 255) / 256));
     const int two_level = sc->host.num_instances ? (sc->host.num_shapes ? 2 : 1) : 0;
     const crt_dev_scene* dsc = (const crt_dev_scene*)ctx->scene_table.p;
-    DevBuf dr, dh, di, dro, drd, dids, dctl;   // until the results are here
-    std::vector<float> po, pd;
     if (flags & CRT_TRACE_STAGE) {
         // the render's closest-hit stage: path-state rays (origin, time 0; direction, depth 1 and the
         // camera bit), one uniform scene, the stage's control words

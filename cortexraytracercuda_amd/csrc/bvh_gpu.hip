@@ -501,10 +501,7 @@ int gpu_build_scene(Context& C, const crt_scene_desc* d, uint32_t leaf, uint32_t
     DevBuf plo, phi, keys[2], vals[2], cb, cl, cr, nlo, nhi, first, count, tmask, tflags, ranks, slot_b, level_base,
         counters, sah, nodes_tmp, tmp, srcmap;
     std::vector<uint32_t> lb, srch;   // read back
-    struct Drain {   // behind every buffer: none goes back while work on it is still queued, on error returns as well
-        hipStream_t s;
-        ~Drain() { (void)hipStreamSynchronize(s); }
-    } drain{s};
+    const StreamDrain drain(s);
     // work buffers come from and return to the context's cache (an allocation and its free cost 0.1-0.4 ms
     // each, and a build takes thirty); large ones at their own size (the cache's classes are powers of two)
     auto work = [&](DevBuf& b, size_t bytes) { return bytes <= (256ull << 20) ? b.alloc_cached(bytes, ctx) : b.alloc(bytes, ctx); };

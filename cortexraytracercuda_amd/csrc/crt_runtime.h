@@ -55,6 +55,16 @@ struct DevBuf {
     ~DevBuf() { release(); }
 };
 
+// Declared behind a call's buffers, so that it goes first: none of them returns to the cache, which other
+// streams take from, while work on it is still queued; on error returns as well.
+struct StreamDrain {
+    hipStream_t s;
+    explicit StreamDrain(hipStream_t st) : s(st) {}
+    StreamDrain(const StreamDrain&) = delete;
+    StreamDrain& operator=(const StreamDrain&) = delete;
+    ~StreamDrain() { (void)hipStreamSynchronize(s); }
+};
+
 struct DeviceScene {
     HostScene host;  // geometry arrays are dropped after upload; stats and small tables stay
     DevBuf geo;   // BVH nodes, then triangle, instance, sphere and quad records (HostScene offsets)

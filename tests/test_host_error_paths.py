@@ -21,3 +21,23 @@ def test_a_device_build_that_fails_leaves_nothing_queued(standin, normals):
             with pytest.raises(A.CrtError, match="injected"):
                 r.upload(s)
             assert standin.standin_pending() == 0, n
+
+
+@pytest.mark.parametrize("stage", [False, True])
+@pytest.mark.parametrize("n", [3, 100001])   # rays that go through the pinned ring, and beyond it
+def test_a_ray_query_that_fails_leaves_nothing_queued(standin, stage, n):
+    rays = np.ones((n, 8), np.float32)
+    with Renderer(max_paths=4096, pass_paths=4096) as r:
+        sid = r.upload(scenes.box_scene())
+        for k in range(2 if stage else 1):   # closest hits, report
+            standin.standin_fail_launch(k)
+            with pytest.raises(A.CrtError, match="launch failed"):
+                r.trace_rays(sid, rays, stage=stage)
+            assert standin.standin_pending() == 0, k
+    with Renderer(max_paths=4096, pass_paths=4096) as r:
+        sid = r.upload(scenes.box_scene())
+        for k in range(7 if stage else 2):   # one buffer after the other, those before it from the cache
+            r.lib.crt_debug_fail_alloc(r.h, min(k, 1))
+            with pytest.raises(A.CrtError, match="injected"):
+                r.trace_rays(sid, rays, stage=stage)
+            assert standin.standin_pending() == 0, k
