@@ -1031,6 +1031,7 @@ int Context::render_noalloc(crt_scene_id scene, const crt_render_desc* rd, float
     PassBufs B;
     if ((rc = scratch_bufs(B))) return rc;
     Job j;
+    PassDrain drain(*this);
     j.setup_external(sc, *rd, accum_dev);
     if (crt_k_init_request(stream, (float4*)accum_dev, nullptr, rd->width, rd->height, rd->seed))
         return set_error(CRT_ERR_HIP, "init kernel launch failed");
@@ -1039,7 +1040,7 @@ int Context::render_noalloc(crt_scene_id scene, const crt_render_desc* rd, float
     if (rgb_dev && crt_k_tonemap(stream, (const float4*)accum_dev, j.npix, rd->spp, rgb_dev))
         return set_error(CRT_ERR_HIP, "tonemap launch failed");
     HIP_TRY(hipStreamSynchronize(stream));
-    return CRT_OK;
+    return drain.done(CRT_OK);
 }
 
 }  // namespace crt
@@ -1140,6 +1141,7 @@ int crt_render_batch(crt_context* c, crt_batch_item* items, uint32_t n, crt_stat
     }
     std::vector<std::unique_ptr<Job>> jobs;
     std::vector<Job*> jp;
+    PassDrain drain(*ctx);
     for (uint32_t k = 0; k < n; ++k) {
         auto j = std::make_unique<Job>();
         int rc = j->setup(ctx, scs[k], items[k].rd);
@@ -1148,7 +1150,7 @@ int crt_render_batch(crt_context* c, crt_batch_item* items, uint32_t n, crt_stat
         jobs.push_back(std::move(j));
     }
     bool time_stages = (n > 0) && (items[0].rd.flags & CRT_RENDER_TIME_STAGES);
-    return ctx->render_jobs(jp, time_stages, stats, ctx->pool_bufs(), items);
+    return drain.done(ctx->render_jobs(jp, time_stages, stats, ctx->pool_bufs(), items));
 }
 
 int crt_trace_rays(crt_context* c, crt_scene_id s, const float* rays, uint64_t n, int32_t flags, int32_t* prim,

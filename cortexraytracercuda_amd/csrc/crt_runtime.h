@@ -358,6 +358,22 @@ struct Context {
     void server_drop_graphs();
 };
 
+// Declared behind the jobs of a blocking call: when the call fails, waits for every stream its passes may
+// have reached before the jobs' buffers go back to the cache (or, a caller's own, to the caller).
+struct PassDrain {
+    Context& c;
+    bool failed = true;
+    explicit PassDrain(Context& ctx) : c(ctx) {}
+    PassDrain(const PassDrain&) = delete;
+    PassDrain& operator=(const PassDrain&) = delete;
+    int done(int rc) { failed = rc != CRT_OK; return rc; }
+    ~PassDrain() {
+        if (!failed) return;
+        (void)hipStreamSynchronize(c.stream);
+        for (hipStream_t s : c.sub_stream) (void)hipStreamSynchronize(s);
+    }
+};
+
 // Both context locks in their order (blocking calls that also change or walk the scene table).
 struct ExecLock {
     std::lock_guard<std::mutex> e, g;

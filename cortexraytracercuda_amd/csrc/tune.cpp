@@ -35,6 +35,7 @@ int Context::tune_trial(crt_scene_id scene, const crt_render_desc& rd, double& m
     DeviceScene* sc = find_scene(scene);
     if (!sc) return set_error(CRT_ERR_INVALID_ARGUMENT, "unknown scene id");
     Job j;
+    PassDrain drain(*this);
     int rc = j.setup(this, sc, rd);
     if (rc) return rc;
     std::vector<Job*> jobs{&j};
@@ -42,7 +43,7 @@ int Context::tune_trial(crt_scene_id scene, const crt_render_desc& rd, double& m
     if ((rc = render_jobs(jobs, false, &st, pool_bufs()))) return rc;
     HIP_TRY(hipStreamSynchronize(stream));
     mrays_s = st.gpu_ms > 0.0 ? (double)st.rays / (st.gpu_ms * 1e-3) / 1e6 : 0.0;
-    return CRT_OK;
+    return drain.done(CRT_OK);
 }
 
 int Context::autotune(crt_scene_id scene, const crt_scene_desc* desc, const crt_render_desc* rd, crt_tune_result* out) {

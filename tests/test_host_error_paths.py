@@ -41,3 +41,31 @@ def test_a_ray_query_that_fails_leaves_nothing_queued(standin, stage, n):
             with pytest.raises(A.CrtError, match="injected"):
                 r.trace_rays(sid, rays, stage=stage)
             assert standin.standin_pending() == 0, k
+
+
+def _batch(sids, n):
+    return [dict(sid=sids[k % len(sids)], width=40 + k, height=30, spp=4, max_depth=3, seed=k, rng=("pcg", "minstd")[k % 2])
+            for k in range(n)]
+
+
+def test_a_batch_that_fails_leaves_nothing_queued(standin):
+    """A launch that is refused while others are queued on the second stream; a request whose buffers cannot
+    be had while the ones before it have theirs started."""
+    with Renderer(max_paths=1 << 14, pass_paths=1 << 14) as r:
+        sids = [r.upload(s) for s in (scenes.box_scene(), scenes.shapes_scene())]
+        for k in range(1, 5):
+            standin.standin_fail_launch(k)
+            with pytest.raises(A.CrtError, match="launch failed"):
+                r.render_batch(_batch(sids, 6))
+            assert standin.standin_pending() == 0, k
+        for k in (1, 3, 7):
+            r.lib.crt_debug_fail_alloc(r.h, k)
+            with pytest.raises(A.CrtError, match="injected"):
+                r.render_batch([dict(j, width=900 + 100 * k, height=600 + 100 * k) for j in _batch(sids, 9)])
+            assert standin.standin_pending() == 0, k
+        _, st = r.render_batch(_batch(sids, 6))
+        assert st["paths"] == sum(j["width"] * j["height"] * 4 for j in _batch(sids, 6))
+        standin.standin_fail_launch(0)
+        with pytest.raises(A.CrtError, match="launch failed"):
+            r.autotune(sids[0], 40, 30, 4, 3)
+        assert standin.standin_pending() == 0
