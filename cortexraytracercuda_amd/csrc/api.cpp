@@ -52,6 +52,9 @@ int DevBuf::alloc(size_t n, Context* ctx) {
         if (left < 0) ctx->fail_alloc_after.store(-1);
     }
     hipError_t e = hipMalloc(&p, n);
+    // what the cache holds is given up before a request, a scene or a query is refused
+    if (e != hipSuccess && ctx && ctx->cache_trim(0)) e = hipMalloc(&p, n);
+    (void)hipGetLastError();   // reported here, not by the next launch
     if (e != hipSuccess) { p = nullptr; return set_error(CRT_ERR_OUT_OF_MEMORY, std::string("hipMalloc: ") + hipGetErrorString(e)); }
     bytes = n;
     return CRT_OK;
@@ -99,6 +102,22 @@ bool Context::cache_put(void* q, size_t cls) {
     buf_cache.emplace(cls, q);
     cache_bytes += cls;
     return true;
+}
+
+// Frees cached buffers, the largest first, until at most `keep` bytes are left; true when it freed any.
+bool Context::cache_trim(size_t keep) {
+    std::vector<void*> out;
+    {
+        std::lock_guard<std::mutex> g(cache_mutex);
+        while (cache_bytes > keep) {
+            auto it = std::prev(buf_cache.end());
+            out.push_back(it->second);
+            cache_bytes -= it->first;
+            buf_cache.erase(it);
+        }
+    }
+    for (void* q : out) (void)hipFree(q);
+    return !out.empty();
 }
 
 template <class T> static int upload_vec(DevBuf& b, const std::vector<T>& v, Context* ctx, hipStream_t s) {

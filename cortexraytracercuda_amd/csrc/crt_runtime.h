@@ -275,6 +275,7 @@ struct Context {
     size_t cache_bytes = 0;
     void* cache_take(size_t cls);
     bool cache_put(void* p, size_t cls);
+    bool cache_trim(size_t keep);
     crt_work_counters last{};        // counters of the last blocking render
 
     // serving
