@@ -77,42 +77,46 @@ int DevBuf::alloc_cached(size_t n, Context* ctx) {
         p = q;
         bytes = cls;
     }
+    asked = n;
     home = ctx;
     return CRT_OK;
 }
 
 void DevBuf::release() {
-    if (p && !(home && home->cache_put(p, bytes))) (void)hipFree(p);
-    p = nullptr; bytes = 0; home = nullptr;
+    if (p && !(home && home->cache_put(p, bytes, asked))) (void)hipFree(p);
+    p = nullptr; bytes = asked = 0; home = nullptr;
 }
 
 void* Context::cache_take(size_t cls) {
     std::lock_guard<std::mutex> g(cache_mutex);
     auto it = buf_cache.find(cls);
     if (it == buf_cache.end()) return nullptr;
-    void* q = it->second;
-    buf_cache.erase(it);
+    void* q = it->second.p;
     cache_bytes -= cls;
+    cache_asked -= it->second.asked;
+    buf_cache.erase(it);
     return q;
 }
 
-bool Context::cache_put(void* q, size_t cls) {
+bool Context::cache_put(void* q, size_t cls, size_t asked) {
     std::lock_guard<std::mutex> g(cache_mutex);
-    if (cache_bytes + cls > kCacheBytes) return false;
-    buf_cache.emplace(cls, q);
+    if (cache_bytes + cls > kCacheBytes || cache_asked + asked > cache_room(0)) return false;
+    buf_cache.emplace(cls, Cached{q, asked});
     cache_bytes += cls;
+    cache_asked += asked;
     return true;
 }
 
 // Frees cached buffers, the largest first, until at most `keep` bytes are left; true when it freed any.
-bool Context::cache_trim(size_t keep) {
+bool Context::cache_trim(uint64_t keep) {
     std::vector<void*> out;
     {
         std::lock_guard<std::mutex> g(cache_mutex);
-        while (cache_bytes > keep) {
+        while (cache_asked > keep) {
             auto it = std::prev(buf_cache.end());
-            out.push_back(it->second);
+            out.push_back(it->second.p);
             cache_bytes -= it->first;
+            cache_asked -= it->second.asked;
             buf_cache.erase(it);
         }
     }
@@ -288,7 +292,7 @@ int Context::scratch_bufs(PassBufs& B) {
 }
 
 uint64_t Context::used_bytes() const {
-    uint64_t b = scene_table.bytes + counters.bytes + ctl.bytes + gstack.bytes + req_table[0].bytes + req_table[1].bytes;
+    uint64_t b = scene_table.bytes + counters.bytes + ctl.bytes + path_next.bytes + gstack.bytes + req_table[0].bytes + req_table[1].bytes;
     for (int k = 0; k < 2; ++k) b += ray_o[k].bytes + ray_d[k].bytes + thr[k].bytes + rad[k].bytes + ids[k].bytes;
     b += hit.bytes + hit_inst.bytes + out_rad.bytes;
     return b;
@@ -369,9 +373,7 @@ Context::~Context() {
     if (stream) (void)hipStreamDestroy(stream);
     // every request has completed (stop_server) and every blocking render returned: the cache
     // holds the last per-request buffers
-    for (auto& kv : buf_cache) (void)hipFree(kv.second);
-    buf_cache.clear();
-    cache_bytes = 0;
+    (void)cache_trim(0);
 }
 
 // ------------------------------------------------------------------ scenes
@@ -381,7 +383,7 @@ int Context::upload_scene(const crt_scene_desc* desc, crt_scene_id* out) {
 }
 
 // Device bytes a device build of `d` may take at most (the scene's own allocations; the build's
-// work buffers come and go within the call): one node per binary interior node, every record,
+// work buffers come from the buffer cache and go back to it, beyond 256 MiB each to the device): one node per binary interior node, every record,
 // per-triangle normals / uvs, sphere mappings and the tables.
 static uint64_t device_build_bound(const crt_scene_desc* d, uint32_t width, uint64_t tables) {
     uint64_t nt = 0;
@@ -424,6 +426,7 @@ int Context::upload_scene_locked(const crt_scene_desc* desc, uint32_t leaf, uint
         tables += ((uint64_t)desc->num_materials + desc->num_lights + 2ull * desc->num_sphere_lights + desc->num_shapes) * 32u;
         if (scene_bytes + request_bytes + reserved + device_build_bound(desc, width, tables) > budget)
             return set_error(CRT_ERR_OVER_BUDGET, "scene exceeds the HBM budget");
+        cache_trim(cache_room(device_build_bound(desc, width, tables)));
         int rc = gpu_build_scene(*this, desc, leaf, width, *sc, err);
         if (rc) return err.empty() ? rc : set_error(rc, err);
         need = sc->bytes;
@@ -434,6 +437,7 @@ int Context::upload_scene_locked(const crt_scene_desc* desc, uint32_t leaf, uint
         need = H.device_bytes();
         if (scene_bytes + request_bytes + reserved + need > budget)
             return set_error(CRT_ERR_OVER_BUDGET, "scene of " + std::to_string(need) + " bytes exceeds the HBM budget");
+        cache_trim(cache_room(need));
         t0 = std::chrono::steady_clock::now();
         {
             // nodes, triangle, instance, sphere and quad records in one allocation, in that order (the
@@ -1146,9 +1150,9 @@ int crt_render_batch(crt_context* c, crt_batch_item* items, uint32_t n, crt_stat
     // stay resident: only release_scene frees one, and it takes exec_mutex.
     std::lock_guard<std::mutex> ex(ctx->exec_mutex);
     std::vector<DeviceScene*> scs(n);
+    uint64_t need = 0;
     {
         std::lock_guard<std::mutex> g(ctx->gpu_mutex);
-        uint64_t need = 0;
         for (uint32_t k = 0; k < n; ++k) {
             if (!(scs[k] = ctx->find_scene(items[k].scene))) return set_error(CRT_ERR_INVALID_ARGUMENT, "unknown scene id");
             int rc = Job::validate(items[k].rd);
@@ -1168,6 +1172,7 @@ int crt_render_batch(crt_context* c, crt_batch_item* items, uint32_t n, crt_stat
         jp.push_back(j.get());
         jobs.push_back(std::move(j));
     }
+    ctx->cache_trim(ctx->cache_room(need));   // the buffers are out of it by now
     bool time_stages = (n > 0) && (items[0].rd.flags & CRT_RENDER_TIME_STAGES);
     return drain.done(ctx->render_jobs(jp, time_stages, stats, ctx->pool_bufs(), items));
 }

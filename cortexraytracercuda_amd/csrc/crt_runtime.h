@@ -42,7 +42,7 @@ constexpr uint32_t kDefaultLeafSize = 1, kDefaultBvhWidth = 4;
 
 struct DevBuf {
     void* p = nullptr;
-    size_t bytes = 0;
+    size_t bytes = 0, asked = 0;
     Context* home = nullptr;   // set: the buffer came from (and returns to) the context's cache
     int alloc(size_t n, Context* ctx);
     // per-request buffers: reuse a cached allocation of the same size class (no hipMalloc / hipFree
@@ -225,7 +225,8 @@ struct Context {
     int device = 0;
     int num_cus = 256;
     hipStream_t stream = nullptr;
-    uint64_t budget = 0, reserved = 0, scene_bytes = 0, request_bytes = 0;
+    // changed under gpu_mutex, request_bytes by the serving threads; the buffer cache reads them on any thread
+    std::atomic<uint64_t> budget{0}, reserved{0}, scene_bytes{0}, request_bytes{0};
     uint32_t max_paths = 0, path_capacity = 0, leaf_size = kDefaultLeafSize, bvh_width = kDefaultBvhWidth, extend_grid = 2048, shade_grid = 2048;
     int extend_mode = CRT_EXTEND_GRID_STRIDE;   // closest-hit work distribution (CRT_EXTEND_*)
     uint32_t extend_param = 2;       // lane-refill threshold or 64-ray groups per wave fetch
@@ -268,14 +269,22 @@ struct Context {
     hipEvent_t sub_done[kMaxSubPasses - 1] = {};
     hipEvent_t ev_pass_ready = nullptr;
     std::atomic<int> fail_alloc_after{-1};   // test hook (crt_debug_fail_alloc): fail the n-th next device allocation
-    // released per-request device buffers, by size class (power of two), at most kCacheBytes
+    // released device buffers of requests, ray queries and device builds, by size class (power of two): at
+    // most kCacheBytes, and by the sizes last asked for (as the budget counts them) no more than the
+    // budget leaves beside what is reserved, resident and admitted
     static constexpr size_t kCacheBytes = 4ull << 30;
+    struct Cached { void* p; size_t asked; };
     std::mutex cache_mutex;
-    std::multimap<size_t, void*> buf_cache;
-    size_t cache_bytes = 0;
+    std::multimap<size_t, Cached> buf_cache;
+    size_t cache_bytes = 0, cache_asked = 0;
     void* cache_take(size_t cls);
-    bool cache_put(void* p, size_t cls);
-    bool cache_trim(size_t keep);
+    bool cache_put(void* p, size_t cls, size_t asked);
+    bool cache_trim(uint64_t keep);
+    // bytes the budget leaves for the cache when `need` more are in use
+    uint64_t cache_room(uint64_t need) const {
+        const uint64_t held = reserved + scene_bytes + request_bytes + need, b = budget;
+        return b > held ? b - held : 0;
+    }
     crt_work_counters last{};        // counters of the last blocking render
 
     // serving

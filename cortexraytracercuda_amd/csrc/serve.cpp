@@ -103,6 +103,7 @@ int Context::server_init() {
         if (rc) return rc;
     }
     reserved = used_bytes() + server_bytes();
+    cache_trim(cache_room(0));
     return CRT_OK;
 }
 
@@ -637,10 +638,11 @@ void Context::server_complete(const std::vector<std::pair<ServeReq*, int>>& done
                 r->timing.rays = rays[k];
         }
         if (r->ev_done) { (void)hipEventDestroy(r->ev_done); r->ev_done = nullptr; }
-        // the job's buffers go back to the cache (own lock); its stream work has completed
+        // the job's buffers go back to the cache (own lock), into the room that they leave in the budget; its
+        // stream work has completed
+        request_bytes -= Job::bytes_needed(r->rd);
         r->job.reset();
         std::lock_guard<std::mutex> lk(srv_mutex);
-        request_bytes -= Job::bytes_needed(r->rd);
         r->sc->refs--;
         complete(r, st, srv_done_cv);
         srv_cv.notify_all();   // the budget it held may admit a waiting request
@@ -742,6 +744,7 @@ void Context::server_loop() {
                 srv_active.push_back(r);
             }
         }
+        if (!admitted.empty()) cache_trim(cache_room(0));   // their buffers are out of it by now
         {
             std::lock_guard<std::mutex> lk(srv_mutex);
             act = srv_active;

@@ -147,6 +147,7 @@ int Context::autotune(crt_scene_id scene, const crt_scene_desc* desc, const crt_
         extend_param = s.param;
         stack_lds = s.lds;
         reserved = used_bytes() + server_bytes();
+        cache_trim(cache_room(0));
         return CRT_OK;
     };
     auto sweep = [&](auto field_set, std::initializer_list<uint32_t> values) -> int {
