@@ -318,7 +318,7 @@ struct Context {
     int ensure_gstack(uint32_t blocks);
     uint64_t server_bytes() const;
     int autotune(crt_scene_id scene, const crt_scene_desc* desc, const crt_render_desc* rd, crt_tune_result* out);
-    int tune_trial(crt_scene_id scene, const crt_render_desc& rd, double& mrays_s);
+    int tune_trial(crt_scene_id scene, const crt_render_desc& rd, double& mrays_s, uint32_t n = 1);
     int trial_scene(crt_scene_id scene, const crt_render_desc& rd, double& mrays_s, uint32_t& trials);
     crt_paths paths(int k, uint32_t slot0);
     int upload_scene(const crt_scene_desc* desc, crt_scene_id* out);

@@ -6,7 +6,8 @@
 // the closest-hit work distribution and traversal stack depth, and on the BVH (width, leaf size).
 // The best values differ between scenes and image sizes, so crt_autotune measures: it times trial
 // renders of the caller's request (full image, a sample range sized to fill the largest slot pool
-// twice) for each candidate of one tunable at a time, keeping the others at their best so far.
+// twice) for each candidate of one tunable at a time, keeping the others at their best so far. Whole-path
+// launches have no such shape: there the BVH and the streams that requests go round are tuned.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -17,6 +18,9 @@
 namespace crt {
 
 namespace {
+
+constexpr uint32_t kTuneRequests = 8;   // renders of a trial of the streams
+constexpr double kTuneGain = 1.05;      // what their slower trial must gain over the faster one so far
 
 struct Shape {
     uint32_t slots, grid, sgrid, sub, mode, param, lds;
@@ -29,16 +33,19 @@ Shape current_shape(const Context& c) {
 
 }  // namespace
 
-// One timed trial render of `rd` on `scene` with the context's current shape (caller holds
+// One timed trial of `n` renders of `rd` on `scene` with the context's current shape (caller holds
 // both context locks). Throughput = closest-hit queries / GPU time of the passes.
-int Context::tune_trial(crt_scene_id scene, const crt_render_desc& rd, double& mrays_s) {
+int Context::tune_trial(crt_scene_id scene, const crt_render_desc& rd, double& mrays_s, uint32_t n) {
     DeviceScene* sc = find_scene(scene);
     if (!sc) return set_error(CRT_ERR_INVALID_ARGUMENT, "unknown scene id");
-    Job j;
+    std::vector<Job> each(n);
+    std::vector<Job*> jobs;
     PassDrain drain(*this);
-    int rc = j.setup(this, sc, rd);
-    if (rc) return rc;
-    std::vector<Job*> jobs{&j};
+    int rc;
+    for (Job& j : each) {
+        if ((rc = j.setup(this, sc, rd))) return rc;
+        jobs.push_back(&j);
+    }
     crt_stats st{};
     if ((rc = render_jobs(jobs, false, &st, pool_bufs()))) return rc;
     HIP_TRY(hipStreamSynchronize(stream));
@@ -121,7 +128,8 @@ int Context::autotune(crt_scene_id scene, const crt_scene_desc* desc, const crt_
         sc = find_scene(scene);
     }
 
-    // whole-path launches (four-wide scenes) have one tunable, their streams; the others belong to the stages
+    // whole-path launches (four-wide scenes) have one tunable, the streams that the requests of a call go
+    // round; the others belong to the stages
     const bool stages = staged || sc->host.bvh_width != 4;
 
     // launch and memory shape, one tunable at a time
@@ -168,7 +176,40 @@ int Context::autotune(crt_scene_id scene, const crt_scene_desc* desc, const crt_
     if (stages && (rc = sweep([](Shape& s, uint32_t v) { s.slots = v; }, {1u << 23, 1u << 24, 1u << 25, 1u << 26}))) return rc;
     if (stages && (rc = sweep([](Shape& s, uint32_t v) { s.grid = v; }, {12u, 24u, 32u}))) return rc;
     if (stages && (rc = sweep([](Shape& s, uint32_t v) { s.sgrid = v; }, {4u, 8u, 16u}))) return rc;
-    if ((rc = sweep([](Shape& s, uint32_t v) { s.sub = v; }, {1u, 2u, 3u, 4u}))) return rc;
+    if (stages && (rc = sweep([](Shape& s, uint32_t v) { s.sub = v; }, {1u, 2u, 3u, 4u}))) return rc;
+    if (!stages) {
+        // one request is one launch, whatever the streams: timed with several, of fewer samples each. The
+        // streams also set the serving loop's lanes, so others are taken only for more than the trials differ
+        crt_render_desc part = tr;
+        if (tr.rng_mode == CRT_RNG_PCG) part.sample_count = std::max(1u, want / kTuneRequests);
+        const uint64_t used = reserved + scene_bytes + request_bytes, room = budget > used ? budget - used : 0;
+        const uint32_t n = (uint32_t)std::min<uint64_t>(kTuneRequests, room / Job::bytes_needed(part));
+        const uint32_t first = bs.sub;
+        double most = 0.0;
+        auto timed = [&](uint32_t sub, double& worse, double& better) -> int {
+            Shape s = bs;
+            s.sub = sub;
+            int r = apply(s);
+            double a = 0.0, b = 0.0;
+            if (r || (r = tune_trial(scene, part, a, n)) || (r = tune_trial(scene, part, b, n))) return r;
+            trials += 2;
+            worse = std::min(a, b);
+            better = std::max(a, b);
+            return CRT_OK;
+        };
+        double worse;
+        if (n > 1) {
+            if ((rc = timed(first, worse, most))) return rc;   // first use of these sizes
+            if ((rc = timed(first, worse, most))) return rc;
+            for (uint32_t v = 1; v <= (uint32_t)kMaxSubPasses; ++v) {
+                double better;
+                if (v == first) continue;
+                if ((rc = timed(v, worse, better))) return rc;
+                if (worse > kTuneGain * most) { most = better; bs.sub = v; }
+            }
+            if ((rc = apply(bs))) return rc;
+        }
+    }
     // closest-hit work distribution: grid-stride (coherent waves) or per-lane refill from the
     // wave's share of the queue after 16 / 32 idle lanes (fewer idle lanes on long, uneven rays)
     if (stages && (rc = sweep(
