@@ -297,6 +297,7 @@ struct Context {
     bool srv_copy_stop = false;
     std::thread srv_thread;
     bool srv_running = false, srv_stop = false;
+    std::atomic<uint64_t> srv_news{0};                 // grows with whatever the scheduler has to look at
     std::deque<ServeReq*> srv_waiting;                 // submitted, not admitted
     std::vector<ServeReq*> srv_active;                 // admitted, on the device
     std::map<crt_request_id, std::unique_ptr<ServeReq>> srv_all;
@@ -360,7 +361,8 @@ struct Context {
     int launch_group(uint32_t lane, std::vector<std::pair<ServeReq*, WorkItem>>& group);
     int finish_whole(uint32_t lane, ServeReq* r);
     int after_others(uint32_t lane, const ServeReq* r);
-    int land_launches(bool wait, bool& any_step);
+    int land_launches(bool& any_step);
+    int await_launch(uint64_t seen);
     bool append_segment(Server& S, ServeReq* r, uint32_t seg_cap);
     int server_process_snapshot(Server& S, std::vector<ServeReq*>& act);
     void server_reset_pass(Server& S);

@@ -26,7 +26,10 @@
 //   - when a pass has no room left (path ids or table entries) it drains and starts over.
 // Results do not depend on the mix: streams are keyed per (seed, pixel, sample, bounce) and each
 // pixel's samples are summed in sample order whatever the segment boundaries are.
+#include <sys/prctl.h>
+
 #include <algorithm>
+#include <chrono>
 #include <cstring>
 
 #include "crt_kernels.h"
@@ -65,6 +68,7 @@ int Context::submit(crt_scene_id scene, const crt_render_desc* rd, crt_request_i
     *out = r->id;
     srv_waiting.push_back(r.get());
     srv_all[r->id] = std::move(r);
+    srv_news++;
     if (!srv_running) {
         srv_running = true;
         srv_stop = false;
@@ -79,6 +83,7 @@ void Context::stop_server() {
         std::lock_guard<std::mutex> lk(srv_mutex);
         if (!srv_running) return;
         srv_stop = true;
+        srv_news++;
         for (ServeReq* r : srv_waiting) r->cancel = true;
         for (ServeReq* r : srv_active) r->cancel = true;
     }
@@ -587,14 +592,8 @@ int Context::launch_whole(const std::vector<ServeReq*>& act, bool& any_step) {
     }
 }
 
-// Takes finished launches off the lanes; `wait`: the one that the emptiest lane will finish next.
-int Context::land_launches(bool wait, bool& any_step) {
-    if (wait) {
-        int best = -1;
-        for (uint32_t l = 0; l < srv_lanes; ++l)
-            if (srv[l].landed < srv[l].launched && (best < 0 || srv[l].ids_ahead < srv[best].ids_ahead)) best = (int)l;
-        if (best >= 0) HIP_TRY(hipEventSynchronize(srv[best].ev[srv[best].landed % Server::kRing]));
-    }
+// Takes finished launches off the lanes.
+int Context::land_launches(bool& any_step) {
     for (uint32_t l = 0; l < srv_lanes; ++l) {
         Server& S = srv[l];
         while (S.landed < S.launched) {
@@ -604,6 +603,25 @@ int Context::land_launches(bool wait, bool& any_step) {
             S.ids_ahead -= S.launch_ids[S.landed % Server::kRing];
             S.landed++;
             any_step = true;
+        }
+    }
+    return CRT_OK;
+}
+
+// Waits until a launch has landed or there is news since `seen` (a request, a cancellation, a completion, the
+// end): a launch takes up to some ten milliseconds, and an idle lane can take a new request meanwhile. Short
+// launches are awaited by polling alone, longer ones between sleeps (the thread's timer slack is 1 us).
+int Context::await_launch(uint64_t seen) {
+    const double t0 = now_s();
+    while (srv_news.load() == seen) {
+        bool any = false;
+        const int rc = land_launches(any);
+        if (rc || any) return rc;
+        if (now_s() - t0 < 200e-6) {
+            std::this_thread::yield();
+        } else {
+            std::unique_lock<std::mutex> lk(srv_mutex);
+            srv_cv.wait_for(lk, std::chrono::microseconds(20), [&]() { return srv_news.load() != seen; });
         }
     }
     return CRT_OK;
@@ -645,6 +663,7 @@ void Context::server_complete(const std::vector<std::pair<ServeReq*, int>>& done
         std::lock_guard<std::mutex> lk(srv_mutex);
         r->sc->refs--;
         complete(r, st, srv_done_cv);
+        srv_news++;
         srv_cv.notify_all();   // the budget it held may admit a waiting request
     }
 }
@@ -671,6 +690,7 @@ void Context::server_copy_loop() {
 void Context::server_loop() {
     const uint32_t L = srv_lanes;
     int err = CRT_OK;
+    (void)prctl(PR_SET_TIMERSLACK, 1000ul, 0, 0, 0);   // this thread's sleeps are short
     {
         std::lock_guard<std::mutex> lk(srv_mutex);
         srv_copy_stop = false;
@@ -687,8 +707,10 @@ void Context::server_loop() {
     for (;;) {
         std::vector<ServeReq*> admitted, act;
         const bool inflight = lanes_inflight();
+        uint64_t news;
         {
             std::unique_lock<std::mutex> lk(srv_mutex);
+            news = srv_news.load();
             const bool work = lanes_work();
             srv_cv.wait(lk, [&]() { return srv_stop || !srv_waiting.empty() || !srv_active.empty() || inflight || work; });
             // drop cancelled waiting requests
@@ -753,9 +775,9 @@ void Context::server_loop() {
         std::vector<ServeReq*> lane_act[kSrvLanes];
         const bool whole = serve_whole();
         if (whole) {
-            err = land_launches(false, any_step);
+            err = land_launches(any_step);
             if (!err) err = launch_whole(act, any_step);
-            if (!err && !any_step) err = land_launches(true, any_step);
+            if (!err && !any_step && lanes_inflight()) err = await_launch(news);
             busy = busy || lanes_inflight();
         }
         for (uint32_t l = 0; l < L && !err && !whole; ++l) {
@@ -891,6 +913,7 @@ int crt_cancel(crt_context* c, crt_request_id req) {
     auto it = ctx->srv_all.find(req);
     if (it == ctx->srv_all.end()) return set_error(CRT_ERR_INVALID_ARGUMENT, "unknown request id");
     it->second->cancel = true;
+    ctx->srv_news++;
     ctx->srv_cv.notify_all();
     return CRT_OK;
 }

@@ -1,0 +1,51 @@
+"""The serving loop's scheduler while launches run that do not end. On the CPU (hip_standin), where path
+launches wait at a gate."""
+import time
+
+import numpy as np
+import pytest
+
+from cortexraytracercuda_amd import Renderer, _abi as A, scenes
+from hip_standin import gate_closed, launches_that_ran, standin, standin_lib  # noqa: F401
+
+
+def _until(what, seconds=10.0):
+    end = time.monotonic() + seconds
+    while time.monotonic() < end:
+        if what():
+            return True
+        time.sleep(0.002)
+    return False
+
+
+def test_a_request_that_arrives_during_a_launch_takes_the_idle_lane(standin):
+    with Renderer(max_paths=1 << 15, pass_paths=1 << 16) as r:
+        sid = r.upload(scenes.box_scene())
+        with gate_closed(standin):
+            first = r.submit(sid, 64, 64, 4, 3, seed=1)
+            assert _until(lambda: standin.standin_launches() == 1)
+            time.sleep(0.05)   # the scheduler has nothing left to do
+            second = r.submit(sid, 8, 8, 4, 3, seed=2)
+            assert _until(lambda: standin.standin_launches() == 2)
+            assert not r.poll(first) and not r.poll(second)
+        for i, w in ((first, 64), (second, 8)):
+            assert r.wait(i, w, w)[2]["rays"] == w * w * 4
+
+
+def test_a_waiting_request_is_cancelled_during_a_launch(standin):
+    with Renderer(max_paths=1 << 15, pass_paths=1 << 16) as r:
+        r.wait(r.submit(r.upload(scenes.box_scene()), 8, 8, 1, 2), 8, 8)
+        held = sum(r.memory()[k] for k in ("reserved", "scenes"))
+    with Renderer(max_paths=1 << 15, pass_paths=1 << 16, hbm_budget=held + 64 * 64 * 19 + 4096) as r:
+        sid = r.upload(scenes.box_scene())
+        with gate_closed(standin):
+            first = r.submit(sid, 64, 64, 4, 3, seed=1)
+            assert _until(lambda: standin.standin_launches() == 1)
+            time.sleep(0.05)
+            second = r.submit(sid, 64, 60, 4, 3, seed=2)   # does not fit beside the first
+            r.cancel(second)
+            assert _until(lambda: r.poll(second))
+            with pytest.raises(A.CrtError, match="cancelled"):
+                r.wait(second, 64, 60)
+            assert not r.poll(first)
+        assert r.wait(first, 64, 64)[2]["rays"] == 64 * 64 * 4
