@@ -660,14 +660,14 @@ bool Job::take(uint32_t cap, WorkItem& w) {
     return true;
 }
 
-bool Job::take_whole(uint32_t cap, WorkItem& w) {
+bool Job::take_whole(uint32_t cap, WorkItem& w, uint32_t samples) {
     if (rd.rng_mode != CRT_RNG_MINSTD) return take(cap, w);
     if (s_next >= s_end || cap == 0) return false;
     w.job = this;
     w.pix_begin = p_next; w.pix_count = std::min(cap, npix - p_next);
-    w.sample_begin = s_next; w.sample_count = s_end - s_next;
+    w.sample_begin = s_next; w.sample_count = std::min(samples, s_end - s_next);
     p_next += w.pix_count;
-    if (p_next == npix) { p_next = 0; s_next = s_end; }
+    if (p_next == npix) { p_next = 0; s_next += w.sample_count; }
     return true;
 }
 

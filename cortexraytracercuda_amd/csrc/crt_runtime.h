@@ -136,8 +136,9 @@ struct Job {
     // a job whose accumulation buffer the caller owns (device memory): no allocation
     void setup_external(DeviceScene* sc, const crt_render_desc& r, float* accum_dev);
     bool take(uint32_t cap, WorkItem& w);
-    // the same for a whole-path launch: a MINSTD job gives pixels with all of their samples
-    bool take_whole(uint32_t cap, WorkItem& w);
+    // the same for a whole-path launch: a MINSTD job gives pixels with the next `samples` of theirs (the same
+    // number in every call), or all
+    bool take_whole(uint32_t cap, WorkItem& w, uint32_t samples = UINT32_MAX);
     bool scheduled_all() const { return s_next >= s_end; }
     // path ids not yet handed to a pass
     uint64_t paths_left() const { return s_next >= s_end ? 0 : (uint64_t)(s_end - s_next) * npix - p_next; }
@@ -305,9 +306,9 @@ struct Context {
     // up to kSrvLanes open passes on their own streams (each with a share of the slot pool), so one
     // pass's drain tail overlaps the other's full launches; a request's segments stay in one lane
     static constexpr int kSrvLanes = 2;
-    // path ids of one whole-path launch of the serving loop, at least for MINSTD, whose ids are pixels;
-    // a lane with kServeAhead of them gets no more
-    static constexpr uint32_t kServeLaunch = 1u << 23, kServeStreams = 1u << 18, kServeAhead = 1u << 23;
+    // path ids of one whole-path launch of the serving loop, at least for MINSTD, whose ids are pixels with
+    // at most kServeSamples samples one after the other; a lane with kServeAhead path ids gets no more
+    static constexpr uint32_t kServeLaunch = 1u << 23, kServeStreams = 1u << 18, kServeSamples = 64, kServeAhead = 1u << 23;
     Server srv[kSrvLanes];
     uint32_t srv_lanes = 1;
     uint64_t lane_load[kSrvLanes] = {};

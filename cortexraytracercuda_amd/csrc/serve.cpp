@@ -506,6 +506,8 @@ int Context::launch_group(uint32_t lane, std::vector<std::pair<ServeReq*, WorkIt
         } else if (!(r->lanes_seen >> lane & 1u)) {
             HIP_TRY(hipStreamWaitEvent(S.s, r->ev_done, 0));
         }
+        // a MINSTD pixel goes on from where its samples before, on whichever lane, left its engine and sums
+        if (q.rng_mode == CRT_RNG_MINSTD && w.sample_begin > r->job->s_begin && (rc = after_others(lane, r))) return rc;
         r->lanes_seen |= 1u << lane;
     }
     if (end > S.cap) return set_error(CRT_ERR_INTERNAL, "launch exceeds the lane's path ids");
@@ -572,14 +574,15 @@ int Context::launch_whole(const std::vector<ServeReq*>& act, bool& any_step) {
             const bool stream = r->rd.rng_mode == CRT_RNG_MINSTD;
             WorkItem w;
             if (group.empty()) {
-                // MINSTD: a pixel's samples run in turn, so the launch is bounded by pixels and paths
+                // MINSTD: a pixel's samples run in turn, up to kServeSamples of them (2^24 paths at most); with
+                // fewer the launch has more pixels
                 const uint32_t c = !stream ? cap : std::min(cap, std::max(kServeStreams, kServeLaunch / std::max(1u, j.nsamples)));
-                if (!j.take_whole(c, w)) continue;
+                if (!j.take_whole(c, w, kServeSamples)) continue;
             } else {
                 const uint64_t left = stream ? j.npix - j.p_next : j.paths_left();
                 w.job = &j;
                 if (!w.same_kernel(group[0].second) || whole_span(end) + left > merge) continue;
-                if (!j.take_whole(merge - whole_span(end), w)) continue;
+                if (!j.take_whole(merge - whole_span(end), w, kServeSamples)) continue;
             }
             end = whole_span(end) + w.whole_ids();
             group.emplace_back(r, w);

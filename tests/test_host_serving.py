@@ -49,3 +49,34 @@ def test_a_waiting_request_is_cancelled_during_a_launch(standin):
                 r.wait(second, 64, 60)
             assert not r.poll(first)
         assert r.wait(first, 64, 64)[2]["rays"] == 64 * 64 * 4
+
+
+@pytest.mark.parametrize("w,h,spp,cap", [(16, 12, 1, 0), (16, 12, 64, 0), (16, 12, 81, 0), (31, 17, 1024, 0), (8, 4, 65536, 0),
+                                         (31, 17, 400, 200), (64, 33, 144, 1000)])
+def test_reference_streams_are_served_in_bounded_launches(standin, w, h, spp, cap):
+    """A pixel's samples go on from one launch to the next, on whichever lane: sums equal the blocking
+    render's. With `cap` path ids a lane, pixels are cut as well."""
+    with Renderer(max_paths=max(cap * 2, 1 << 12), pass_paths=max(cap * 2, 1 << 24)) as r:
+        sid = r.upload(scenes.box_scene())
+        rgb, acc, st = r.render(sid, w, h, spp, 3, seed=5, rng="minstd")
+        alone = len(launches_that_ran(standin))
+        others = [r.submit(sid, 20, 10, 9, 3, seed=k, rng=m) for k, m in enumerate(("pcg", "minstd"))]
+        mine = r.submit(sid, w, h, spp, 3, seed=5, rng="minstd")
+        srgb, sacc, sst = r.wait(mine, w, h)
+        for k in others:
+            r.wait(k, 20, 10)
+        assert np.array_equal(sacc, acc) and np.array_equal(srgb, rgb) and sst["rays"] == st["rays"]
+        for l in launches_that_ran(standin)[alone:]:
+            if l["mode"] == A.CRT_RNG_MINSTD:
+                assert l["samples"] <= 64 and l["paths"] <= 1 << 24
+
+
+def test_reference_streams_over_many_pixels_are_served_in_bounded_launches(standin):
+    with Renderer(max_paths=1 << 12, pass_paths=1 << 24) as r:
+        sid = r.upload(scenes.box_scene())
+        _, acc, _ = r.render(sid, 700, 500, 81, 3, seed=5, rng="minstd")
+        alone = len(launches_that_ran(standin))
+        _, sacc, _ = r.wait(r.submit(sid, 700, 500, 81, 3, seed=5, rng="minstd"), 700, 500)
+        assert np.array_equal(sacc, acc)
+        ran = launches_that_ran(standin)[alone:]
+        assert len(ran) == 4 and max(l["paths"] for l in ran) <= 1 << 24
