@@ -1191,7 +1191,7 @@ int crt_trace_rays(crt_context* c, crt_scene_id s, const float* rays, uint64_t n
     auto get = [&](DevBuf& b, uint64_t bytes) { return bytes <= (256ull << 20) ? b.alloc_cached(bytes, ctx) : b.alloc(bytes, ctx); };
     DevBuf out, dr, dh, di, dro, drd, dids, dctl;
     std::vector<float> po, pd;
-    const StreamDrain drain(ctx->stream);
+    StreamDrain drain(ctx->stream);
     int rc;
     const bool camera = (flags & CRT_TRACE_CAMERA) != 0;
     if ((rc = get(out, n * 20))) return rc;
@@ -1242,7 +1242,7 @@ int crt_trace_rays(crt_context* c, crt_scene_id s, const float* rays, uint64_t n
                                      {uv, o + n * 12, uv ? n * 8 : 0}};
     HIP_TRY(ctx->stage.fetch(back, 5, ctx->stream));
     if (cnt.stack_overflow) return set_error(CRT_ERR_INTERNAL, "traversal stack overflow");
-    return CRT_OK;
+    return drain.done(CRT_OK);
 }
 
 int crt_trace_primary(crt_context* c, crt_scene_id s, uint32_t W, uint32_t H, int32_t* prim, float* t) {

@@ -501,7 +501,7 @@ int gpu_build_scene(Context& C, const crt_scene_desc* d, uint32_t leaf, uint32_t
     DevBuf plo, phi, keys[2], vals[2], cb, cl, cr, nlo, nhi, first, count, tmask, tflags, ranks, slot_b, level_base,
         counters, sah, nodes_tmp, tmp, srcmap;
     std::vector<uint32_t> lb, srch;   // read back
-    const StreamDrain drain(s);
+    StreamDrain drain(s);
     // work buffers come from and return to the context's cache (an allocation and its free cost 0.1-0.4 ms
     // each, and a build takes thirty); large ones at their own size (the cache's classes are powers of two)
     auto work = [&](DevBuf& b, size_t bytes) { return bytes <= (256ull << 20) ? b.alloc_cached(bytes, ctx) : b.alloc(bytes, ctx); };
@@ -715,7 +715,7 @@ int gpu_build_scene(Context& C, const crt_scene_desc* d, uint32_t leaf, uint32_t
                sc.texs.bytes + sc.texels.bytes + sc.lights.bytes;
     // the host copies of the tables are not needed after the upload
     H.texels.clear(); H.texels.shrink_to_fit();
-    return CRT_OK;
+    return drain.done(CRT_OK);
 }
 
 }  // namespace crt
