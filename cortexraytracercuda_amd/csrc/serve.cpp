@@ -484,7 +484,8 @@ int Context::launch_group(uint32_t lane, std::vector<std::pair<ServeReq*, WorkIt
     const size_t e0 = (size_t)slot * Server::kLaunchEntries;
     crt_dev_request* dreq = (crt_dev_request*)S.req.p + e0;
     uint32_t end = 0, max_pix = 0;
-    uint64_t ids = 0;
+    uint64_t ids = 0, pixels = 0;
+    uint32_t samples = 0;
     int rc;
     for (size_t k = 0; k < group.size(); ++k) {
         ServeReq* r = group[k].first;
@@ -498,6 +499,8 @@ int Context::launch_group(uint32_t lane, std::vector<std::pair<ServeReq*, WorkIt
         end = q.path_base + w.whole_ids();
         max_pix = std::max(max_pix, w.pix_count);
         ids += (uint64_t)w.pix_count * w.sample_count;
+        pixels += w.pix_count;
+        samples = std::max(samples, w.sample_count);
         // the first launch starts the request's buffers, the other lane's launches come behind that
         if (r->segs == 0) {
             if ((rc = r->job->init(S.s))) return rc;
@@ -540,6 +543,8 @@ int Context::launch_group(uint32_t lane, std::vector<std::pair<ServeReq*, WorkIt
     }
     // behind the tonemaps: a landed launch's finished requests can be read back
     HIP_TRY(hipEventRecord(S.ev[slot], S.s));
+    // MINSTD: samples in turn take their time however few the pixels are
+    if (w0.job->rd.rng_mode == CRT_RNG_MINSTD) ids = std::max(ids, std::max<uint64_t>(pixels, kServeStreams) * samples);
     S.launch_ids[slot] = (uint32_t)std::min<uint64_t>(ids, 0xffffffffu);
     S.ids_ahead += S.launch_ids[slot];
     S.launched++;

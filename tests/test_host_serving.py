@@ -80,3 +80,19 @@ def test_reference_streams_over_many_pixels_are_served_in_bounded_launches(stand
         assert np.array_equal(sacc, acc)
         ran = launches_that_ran(standin)[alone:]
         assert len(ran) == 4 and max(l["paths"] for l in ran) <= 1 << 24
+
+
+def test_a_long_reference_stream_is_not_enqueued_far_ahead(standin):
+    """Sample ranges take their time however small the image is: each lane has one of them, and a request
+    that arrives takes its turn behind those."""
+    with Renderer(max_paths=1 << 12, pass_paths=1 << 22, serve_small_paths=1000) as r:
+        sid = r.upload(scenes.box_scene())
+        with gate_closed(standin):
+            first = r.submit(sid, 32, 20, 4096, 3, seed=1, rng="minstd")
+            assert _until(lambda: standin.standin_launches() == 2)
+            second = r.submit(sid, 8, 8, 4, 3, seed=2)
+            time.sleep(0.1)
+            assert standin.standin_launches() == 2
+        r.wait(second, 8, 8)
+        assert launches_that_ran(standin)[2]["mode"] == A.CRT_RNG_PCG
+        r.wait(first, 32, 20)
