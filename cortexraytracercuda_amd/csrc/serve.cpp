@@ -625,7 +625,7 @@ int Context::await_launch(uint64_t seen) {
         bool any = false;
         const int rc = land_launches(any);
         if (rc || any) return rc;
-        if (now_s() - t0 < 200e-6) {
+        if (now_s() - t0 < 2e-3) {
             std::this_thread::yield();
         } else {
             std::unique_lock<std::mutex> lk(srv_mutex);
