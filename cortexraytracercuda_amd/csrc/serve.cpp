@@ -7,7 +7,8 @@
 //     buffers; scenes are already resident and counted at upload);
 //   - an admitted request is cut into segments (pixel range x sample range) of up to 8 M paths; a
 //     segment is one launch that follows its paths to their end, and its resolve, on the lane with
-//     the fewest paths ahead; the next ones are enqueued while fewer than 8 M are.
+//     the fewest paths ahead; the next ones are enqueued while fewer than 8 M are. (A segment of the
+//     reference stream has at least 2^18 pixels and at most 64 samples of each.)
 //     Segments of one request are resolved in sample order by events between the lanes; after the
 //     last one comes the tonemap, and a completion thread reads the image back;
 //   - short segments of several requests share a launch.

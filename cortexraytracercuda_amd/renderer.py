@@ -44,7 +44,7 @@ class Renderer:
                  graphs=0, stack_lds=0, ray_sort=0, bvh_builder="host", batch_group_paths=0, serve_order="small_then_oldest",
                  serve_small_paths=0):
         """bvh_builder: "host" (binned SAH on the CPU) or "device" (linear BVH built on the GPU).
-        batch_group_paths: render_batch gives a request with at least this many path ids left passes
+        batch_group_paths: in stages, render_batch gives a request with at least this many path ids left passes
         of its own scene (0: the library default, 0xffffffff: every pass mixes requests in order).
         serve_order: "small_then_oldest" (requests with at most serve_small_paths path ids left first,
         then the others oldest first) or "round_robin" (one segment per request in turn)."""
@@ -192,7 +192,7 @@ class Renderer:
 
     def trace_rays(self, sid, rays, camera=False, stage=False):
         """Closest hits of n x 8 rays (origin, tmin, direction, tmax). stage=True answers them with the
-        render's closest-hit stage (estimator interval, pass-through of one-sided lights seen from
+        closest-hit stage of renders that run in stages (estimator interval, pass-through of one-sided lights seen from
         behind) instead of the query kernel."""
         rays = np.ascontiguousarray(rays, dtype=np.float32).reshape(-1, 8)
         n = rays.shape[0]

@@ -312,7 +312,8 @@ typedef struct crt_config {
     uint32_t max_paths;         /* live path slots of the streaming passes (path state pools, 164 B each);
                                    0 = 64M */
     uint32_t block_size;        /* threads per block of the stage kernels; 0 = default (256) */
-    uint32_t count_work;        /* 1: use the counting traversal kernel (fills node_visits/prim_tests) */
+    uint32_t count_work;        /* 1: everything runs in stages, with the counting traversal kernel (fills
+                                   node_visits/prim_tests) */
     uint32_t leaf_size;         /* BVH max primitives per leaf (1-8); 0 = default (1) */
     uint32_t bvh_width;         /* children per BVH node, 2 or 4; 0 = default (4) */
     uint32_t extend_kernel;     /* 0 = default: renders and served requests of four-wide scenes follow whole
@@ -324,21 +325,25 @@ typedef struct crt_config {
                                    2 = per-lane refill: a lane whose ray is done takes the next ray of its
                                        wave's contiguous share of the queue (no atomics),
                                    3 = persistent waves taking chunks of 64-ray groups from a work counter */
+    /* refill_min, grid_per_cu, shade_grid_per_cu, stack_lds, ray_sort, graphs and batch_group_paths shape the
+     * stages; whole-path launches do not read them (grid_per_cu still sizes the traversal's overflow stacks) */
     uint32_t refill_min;        /* mode 2: idle lanes of a wave before they take new rays (default 16);
                                    mode 3: 64-ray groups per fetch; 0 = default */
     uint32_t pass_paths;        /* path ids per pass (16 B of radiance each); 0 = min(2^27, 16 * max_paths)
                                    for blocking renders, min(2^29, 32 * max_paths) for the serving loop */
     uint32_t grid_per_cu;       /* workgroups per CU of the closest-hit launches (256 threads each); 0 = 24 */
     uint32_t shade_grid_per_cu; /* workgroups per CU of the regenerate / shade launches; 0 = 16 */
-    uint32_t sub_passes;        /* concurrent sub-passes (one stream each) of a pass, 1-4; 0 = 2 */
+    uint32_t sub_passes;        /* streams of a blocking call, 1-4; 0 = 2: in stages each has a share of the pass
+                                   (a sub-pass), whole-path launches of several requests go round them; the
+                                   serving loop has as many lanes, at most 2 */
     uint32_t graphs;            /* iterations of a serving loop that runs in stages replayed from hipGraphs:
                                    0 = default (on), 1 = on, 2 = off (every iteration launched eagerly) */
     uint32_t stack_lds;         /* traversal stack: LDS ring entries per lane behind the register top entry,
                                    8, 16 or 32; 0 = 16 */
-    uint32_t ray_sort;          /* 1: the shade stage groups each workgroup's surviving paths by direction
+    uint32_t ray_sort;          /* 1: everything runs in stages, and the shade stage groups each workgroup's surviving paths by direction
                                    octant (coherent waves in the next closest-hit launch); 0 / 2: off */
     uint32_t bvh_builder;       /* CRT_BVH_*: where crt_scene_upload builds the BVH; 0 = host */
-    uint32_t batch_group_paths; /* crt_render_batch: a request with at least this many path ids left gets
+    uint32_t batch_group_paths; /* crt_render_batch in stages: a request with at least this many path ids left gets
                                    passes of its own scene (single-scene kernel, one tree in the caches);
                                    smaller remainders share passes; 0 = 2^22, 0xffffffff = always share */
     uint32_t serve_order;       /* CRT_SERVE_*: the order in which the serving loop feeds admitted requests
@@ -416,8 +421,9 @@ int crt_render_noalloc(crt_context* ctx, crt_scene_id scene, const crt_render_de
  * (ox,oy,oz,tmin, dx,dy,dz,tmax). Outputs per ray: global primitive id (-1 = miss), instance
  * (-1 = none), t, and the barycentric / planar coordinates u, v. `flags` (CRT_TRACE_*):
  * CRT_TRACE_CAMERA hides invisible lights as the reference does for depth == max_depth;
- * CRT_TRACE_STAGE answers the queries with the render's closest-hit stage (the configured
- * extend_kernel, with its exact re-trace of undecided triangle tests) instead of the query kernel:
+ * CRT_TRACE_STAGE answers the queries with the closest-hit stage of renders that run in stages (the
+ * configured extend_kernel, with its exact re-trace of undecided triangle tests) instead of the query
+ * kernel; whole-path launches find the same hits with a traversal of their own:
  * the interval is then the estimator's [1e-5, FLT_MAX) whatever tmin / tmax say, and a one-sided
  * light hit from behind is passed through as in the render (core/src/cameras/camera.cuh:179-183). */
 enum { CRT_TRACE_CAMERA = 1, CRT_TRACE_STAGE = 2 };
@@ -471,12 +477,13 @@ typedef struct crt_tune_result {
     double initial_mrays_s;      /* trial throughput of the settings on entry */
 } crt_tune_result;
 /* No counterpart in the reference, which fixes its launch at 16x16-thread blocks
- * (core/src/gpu.cu:2072-2080). Picks the launch and memory shape of the streaming passes for
- * renders like `rd` of `scene` by timing trial renders (a sample range of `rd`, full image) of each
- * candidate, one tunable at a time: live path slots, closest-hit and shade workgroups per CU,
- * sub-passes, closest-hit work distribution, traversal stack depth in LDS. With `desc` (the
- * scene's description, as uploaded) it first rebuilds the scene's BVH at widths 2/4 and leaf sizes
- * 1/2/4 and keeps the fastest in place (same scene id). The choice becomes the context's setting
+ * (core/src/gpu.cu:2072-2080). Picks the launch and memory shape for renders like `rd` of `scene` by
+ * timing trial renders (a sample range of `rd`, full image) of each candidate, one tunable at a time.
+ * With `desc` (the scene's description, as uploaded) it first rebuilds the scene's BVH at widths 2/4 and
+ * leaf sizes 1/2/4 and keeps the fastest in place (same scene id). Where renders run in stages then come
+ * live path slots, closest-hit and shade workgroups per CU, sub-passes, closest-hit work distribution and
+ * traversal stack depth in LDS; where they are whole-path launches only sub_passes, timed with eight
+ * requests and changed for a gain of more than 5 %. The choice becomes the context's setting
  * for later renders and uploads. Blocking; `desc` may be NULL. */
 int crt_autotune(crt_context* ctx, crt_scene_id scene, const crt_scene_desc* desc, const crt_render_desc* rd,
                  crt_tune_result* out);
