@@ -52,9 +52,12 @@ int DevBuf::alloc(size_t n, Context* ctx) {
         if (left < 0) ctx->fail_alloc_after.store(-1);
     }
     hipError_t e = hipMalloc(&p, n);
-    // what the cache holds is given up before a request, a scene or a query is refused
-    if (e != hipSuccess && ctx && ctx->cache_trim(0)) e = hipMalloc(&p, n);
-    (void)hipGetLastError();   // reported here, not by the next launch
+    // what the cache holds is given up before a request, a scene or a query is refused; the error is reported
+    // here, not by the next launch
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        if (ctx && ctx->cache_trim(0) && (e = hipMalloc(&p, n)) != hipSuccess) (void)hipGetLastError();
+    }
     if (e != hipSuccess) { p = nullptr; return set_error(CRT_ERR_OUT_OF_MEMORY, std::string("hipMalloc: ") + hipGetErrorString(e)); }
     bytes = n;
     return CRT_OK;
